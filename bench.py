@@ -81,11 +81,11 @@ def parse():
 #   LU 5x5 with partial pivoting                    120 (FP64 or FP32)
 #   analytic Jacobian (primal 85, rho/u columns 21, velocity columns 5 + 3 x 57)
 #                                                   282 (FP64 or FP32)
-#   row/column equilibration around the FP32 LU      90 FP32
+#   fused Newton step by elimination (fused.hpp)    177 FP64
 #   update bookkeeping (f0, f'0, P += lambda d)      12 FP64
 OPS = {
     "res_exact": 177, "res_fast": 115, "eval_bookkeeping": 24, "fd_quotients": 65,
-    "fd_quotients_fused": 75, "lu": 120, "analytic_jac": 282, "equilibration": 90, "update": 12,
+    "fd_quotients_fused": 75, "lu": 120, "analytic_jac": 282, "newton_step": 177, "update": 12,
 }
 
 
@@ -101,16 +101,13 @@ def path_flops(path, iters, res_evals, nf=5):
                + iters * (OPS["fd_quotients_fused"] + OPS["lu"] + OPS["update"]))
         return f64, 0.0
     if path.startswith("mixed"):
-        f64 = res_evals * (OPS["res_fast"] + OPS["eval_bookkeeping"]) + iters * OPS["update"]
-        f32 = iters * (OPS["analytic_jac"] + OPS["equilibration"] + OPS["lu"])
-        return f64, f32
+        f64 = res_evals * (OPS["res_fast"] + OPS["eval_bookkeeping"]) + iters * (OPS["newton_step"] + OPS["update"])
+        return f64, 0.0
     if path == "analytic_fp64":
         f64 = (res_evals * (OPS["res_exact"] + OPS["eval_bookkeeping"])
                + iters * (OPS["analytic_jac"] + OPS["lu"] + OPS["update"]))
         return f64, 0.0
-    f64 = res_evals * (OPS["res_fast"] + OPS["eval_bookkeeping"]) + iters * OPS["update"]
-    f32 = iters * (OPS["analytic_jac"] + OPS["equilibration"] + OPS["lu"])
-    return f64, f32
+    raise ValueError(f"no operation count for path {path}")
 
 
 PATHS = {
@@ -306,11 +303,11 @@ def main():
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": "f64 residual/update + f32 Jacobian/LU",
+        "dtype": "f64",
         "data": "synthetic (seeded Kerr-Schild zone batch, known roots)",
         "config": {
             "workload": "isolated batched per-zone Newton, ideal MHD, 2^22 zones, MKS a=0.9375, "
-                        "resid<=1e-10 (per-zone normalised); headline = analytic Jacobian + FP32 LU",
+                        "resid<=1e-10 (per-zone normalised); headline = analytic Newton step by elimination in FP64 (opts GRIM_LU_FP32)",
             "zones": n, "newton_unknowns": p.nf, "primitives": p.dof, "semantics": "per_zone",
         },
         "speedup_vs_fd_fp64": head["zone_updates_per_s"] / fd["zone_updates_per_s"],
@@ -639,9 +636,8 @@ def full_step_bench(args):
                        f"(torus closure), WENO5+LLF, {args.torus_steps} steps after 2 warm-up, Newton to "
                        "relative residual 1e-10 (maxNonLinearIter 10); fd_fp64_lockstep = grim's solve loop "
                        "(every zone updated while any zone is unconverged, solve.cpp:75-78), fd_fp64 = the same "
-                       "FD-FP64 algorithm stopping each zone at its own convergence, mixed = analytic Jacobian "
-                       "with FP32 assembly and LU for the first two updates of each zone and FP64 for the "
-                       "compacted stragglers (FP64 residual and update throughout); the *_fast paths run the "
+                       "FD-FP64 algorithm stopping each zone at its own convergence, mixed = the analytic Newton "
+                       "step by elimination in FP64 (opts GRIM_LU_FP32_FP64); the *_fast paths run the "
                        "same Newton with the explicit stage in its fast form (shared reciprocals, fused "
                        "multiply-adds, 40-plane connection; equal to grim's order to rounding), the others with "
                        "the explicit stage in grim's expression order")

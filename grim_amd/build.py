@@ -13,9 +13,8 @@ Flags that matter:
                       in both kinds of translation unit);
   -fno-hip-fp32-correctly-rounded-divide-sqrt
                       *_fast.hip only: FP32 division and square root by the
-                      hardware reciprocal sequences (the FP32 Jacobian and LU
-                      of the mixed path need no correctly rounded quotients;
-                      FP64 arithmetic is unaffected);
+                      hardware reciprocal sequences (FP64 arithmetic is
+                      unaffected);
   -Xclang -target-feature -Xclang -packed-fp32-ops
                       keeps the compiler from emitting packed FP32 math.
 """

@@ -1,5 +1,6 @@
-// Analytic Jacobian of the per-zone residual (ideal MHD and EMHD) and the
-// fast FP64 residual of the mixed-precision Newton path.
+// Analytic Jacobian of the per-zone residual (ideal MHD and EMHD): the dense
+// tangent, its transpose product and the EMHD weights.  The fused solve
+// eliminates the same system without forming it (fused.hpp).
 //
 // Identities used (normal-observer split, beta^i = alpha^2 g^0i,
 // beta_j = g_0j, gamma_ij = g_ij):
@@ -42,8 +43,7 @@
 // guess element's own closure (tau, chi, nu) never enters the residual:
 // only the coefficient element's does, and it is fixed during the solve.
 //
-// The primal quantities are recomputed in the tangent's precision T (float
-// for the mixed path, double for the analytic FP64 path).
+// The primal quantities are recomputed in the tangent's precision T.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -514,148 +514,6 @@ __device__ __forceinline__ void analyticAdjoint(const double* Pd, const ZoneGeom
   for (int j = 0; j < 3; j++) out[U1 + j] = ut_b[j];
   if constexpr (L::COND_ON) out[L::Q] = qt_b;
   if constexpr (L::VISC_ON) out[L::DP] = dpt_b;
-}
-
-// Ideal-MHD entry kept for the kernels that carry no EMHD constants.
-template <class T, class L>
-__device__ __forceinline__ void analyticJacobianIdeal(const double* Pd, const ZoneGeom& Gd,
-                                                      const DevParams& prm, double scale,
-                                                      T (&A)[L::NF][L::NF]) {
-  static_assert(!L::EMHD, "ideal-MHD tangent");
-  ZoneConst<L> c;
-  EmhdWeights ew;
-  analyticJacobian<T, L>(Pd, Gd, prm, scale, c, ew, 1., A);
-}
-
-// Residual of the mixed-precision path (ideal MHD): FP64 throughout, the same
-// mathematics as residual() evaluated through the identities above, with one
-// FP64 division (1/gamma) and one square root per evaluation instead of nine
-// divisions; 1/alpha and mask/dt come in per zone.  Rounding differs from the
-// grim-order residual at the 1e-16 level, far below the 1e-10 tolerance.
-template <class L>
-__device__ __forceinline__ void residualFastIdeal(const double* P, const ZoneGeom& G,
-                                                  const ZoneConst<L>& c, const DevParams& prm,
-                                                  double invAlpha, double scale, double* R) {
-  static_assert(!L::EMHD, "ideal-MHD residual");
-  const double rho = smax(P[RHO], prm.rhoFloor);
-  const double u = smax(P[UU], prm.uFloor);
-  const double ut[3] = {P[U1], P[U2], P[U3]};
-  const double B[3] = {P[L::B1], P[L::B2], P[L::B3]};
-  const double p = (prm.gam - 1.) * u;
-  double utLow[3], BLow[3];
-#pragma unroll
-  for (int i = 0; i < 3; i++) {
-    utLow[i] = G.cov(i + 1, 1) * ut[0] + G.cov(i + 1, 2) * ut[1] + G.cov(i + 1, 3) * ut[2];
-    BLow[i] = G.cov(i + 1, 1) * B[0] + G.cov(i + 1, 2) * B[1] + G.cov(i + 1, 3) * B[2];
-  }
-  const double lor = sqrt(1. + ut[0] * utLow[0] + ut[1] * utLow[1] + ut[2] * utLow[2]);
-  const double u0 = lor * invAlpha;
-  const double invU0 = G.alpha / lor;
-  const double uCov0 = -G.alpha * lor + G.cov(0, 1) * ut[0] + G.cov(0, 2) * ut[1] + G.cov(0, 3) * ut[2];
-  const double b0 = B[0] * utLow[0] + B[1] * utLow[1] + B[2] * utLow[2];
-  const double bCov0 = (G.cov(0, 1) * B[0] + G.cov(0, 2) * B[1] + G.cov(0, 3) * B[2] + b0 * uCov0) * invU0;
-  const double BB = B[0] * BLow[0] + B[1] * BLow[1] + B[2] * BLow[2];
-  const double bsq = (BB + b0 * b0) * invU0 * invU0 + prm.bSqrFloor;
-  const double wu0 = (rho + u + p + bsq) * u0;
-  const double Urho = G.g * (rho * u0);
-  const double T00 = wu0 * uCov0 - b0 * bCov0 + (p + 0.5 * bsq);
-  R[RHO] = (Urho - c.rhs[RHO]) * scale;
-  R[UU] = (G.g * T00 + Urho - c.rhs[UU]) * scale;
-#pragma unroll
-  for (int i = 0; i < 3; i++) {
-    const double bCovi = (BLow[i] + b0 * utLow[i]) * invU0;
-    R[U1 + i] = (G.g * (wu0 * utLow[i] - b0 * bCovi) - c.rhs[U1 + i]) * scale;
-  }
-}
-
-// The EMHD residual of the fused paths: the same rows as residual<L>, with
-// the per-zone constants folded once per zone.  The time-derivative sources
-// are affine in the new element's u_mu and T with the weights of
-// emhdWeights (S_td = sum_mu w_mu (u_mu - u_mu,old) + w_T (T - T_old), the
-// divisions by dt, tau_c, |b|_c and b^2_c taken once), the implicit source is
-// g qTilde / tau_c, and the rows are scaled by 1/dt, the normalisation and
-// the mask by products.  Equal to residual<L> up to rounding.
-template <class L>
-__device__ __forceinline__ void residualFastEmhd(const double* P, const ZoneGeom& G, const ZoneConst<L>& c,
-                                                 const DevParams& prm, const EmhdWeights& ew, double invDt,
-                                                 double* R) {
-  static_assert(L::EMHD, "EMHD residual");
-  Kinematics k;
-  kinematics<L>(P, G, prm, k);
-  Closure cl;
-  closure<L>(P, k, prm, c.alphaC, c.alphaV, c.radius, cl);
-  const double w = k.rho + k.u + k.pressure + k.bSqr;
-  const double qOverB = L::COND_ON ? cl.q / cl.bNorm : 0.;
-  const double dPOverB2 = L::VISC_ON ? cl.deltaP / k.bSqr : 0.;
-  double T0[4];
-#pragma unroll
-  for (int nu = 0; nu < 4; nu++) {
-    double t = w * k.uCon[0] * k.uCov[nu] - k.bCon[0] * k.bCov[nu];
-    if (nu == 0) t += k.pressure + 0.5 * k.bSqr;
-    if constexpr (L::COND_ON) t += qOverB * (k.uCon[0] * k.bCov[nu] + k.bCon[0] * k.uCov[nu]);
-    if constexpr (L::VISC_ON)
-      t -= dPOverB2 * k.bCon[0] * k.bCov[nu] - (cl.deltaP / 3.) * ((nu == 0 ? 1. : 0.) + k.uCon[0] * k.uCov[nu]);
-    T0[nu] = t;
-  }
-  const double s = c.mask * invDt;
-  const double Urho = G.g * (k.rho * k.uCon[0]);
-  R[RHO] = (Urho - c.rhs[RHO]) * s;
-  R[UU] = (G.g * T0[0] + Urho - c.rhs[UU]) * s;
-#pragma unroll
-  for (int i = 1; i < 4; i++) R[UU + i] = (G.g * T0[i] - c.rhs[UU + i]) * s;
-  double du[4];
-#pragma unroll
-  for (int mu = 0; mu < 4; mu++) du[mu] = k.uCov[mu] - c.oldUCov[mu];
-  if constexpr (L::COND_ON) {
-    double std = ew.wQT * (k.temperature - c.oldT);
-#pragma unroll
-    for (int mu = 0; mu < 4; mu++) std += ew.wQ[mu] * du[mu];
-    const double U = G.g * (k.uCon[0] * P[L::Q]);
-    R[L::Q] = ((U - c.rhs[L::Q]) * invDt + 0.5 * ew.gOverTau * P[L::Q] + std) * ew.sQ;
-  }
-  if constexpr (L::VISC_ON) {
-    double std = 0.;
-#pragma unroll
-    for (int mu = 0; mu < 4; mu++) std += ew.wDP[mu] * du[mu];
-    const double U = G.g * (k.uCon[0] * P[L::DP]);
-    R[L::DP] = ((U - c.rhs[L::DP]) * invDt + 0.5 * ew.gOverTau * P[L::DP] + std) * ew.sDP;
-  }
-}
-
-// Row and column equilibration around the FP32 LU: solve (Dr A Dc) y = Dr b,
-// x = Dc y, with Dc = |P_k| (the natural scale of each primitive) and Dr the
-// inverse of each scaled row's largest entry.  The equilibrated matrix is
-// factorised without pivoting: the row swaps of partial pivoting are selects
-// on every entry (a fifth of the issued instructions of the ideal-MHD solve),
-// and on the 2^22-zone Kerr-Schild batch, the EMHD batch and the torus they
-// changed neither the iteration counts, nor the unconverged zones, nor the
-// error against the known roots.  An FP32 step that goes wrong is rejected
-// by the FP64 line search, and the escalating solve finishes such zones with
-// the pivoted FP64 factorisation.
-template <class T, int N>
-__device__ __forceinline__ void equilibratedSolve(T (&A)[N][N], T (&b)[N], const double* P) {
-  T cs[N];
-#pragma unroll
-  for (int k = 0; k < N; k++) {
-    const T a = (T)fabs(P[k]);
-    cs[k] = (a > T(0) && a < T(1e30)) ? a : T(1);
-  }
-#pragma unroll
-  for (int i = 0; i < N; i++) {
-    T m = T(0);
-#pragma unroll
-    for (int k = 0; k < N; k++) {
-      A[i][k] = A[i][k] * cs[k];
-      m = fmax(m, fabs(A[i][k]));
-    }
-    const T r = (m > T(0)) ? lowRecip(m) : T(1);
-#pragma unroll
-    for (int k = 0; k < N; k++) A[i][k] = A[i][k] * r;
-    b[i] = b[i] * r;
-  }
-  luSolve<T, N, false>(A, b);
-#pragma unroll
-  for (int k = 0; k < N; k++) b[k] = b[k] * cs[k];
 }
 
 }  // namespace grim

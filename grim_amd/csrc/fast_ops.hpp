@@ -11,6 +11,9 @@
 //    residual correction of the quotient (within about one ulp of the
 //    correctly rounded result for finite, nonzero, normal divisors; a zero
 //    or infinite divisor gives NaN where IEEE division gives inf or 0).
+//  * fastSqrt / fastRsqrt: square root and its reciprocal from the hardware
+//    estimate with one higher-order refinement (within about one ulp; exact
+//    at zero for fastSqrt; arguments of ordinary magnitude).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -47,6 +50,22 @@ __device__ __forceinline__ double fastDiv(double a, double b) {
   const double r = fastRcp(b);
   const double q = a * r;
   return __builtin_fma(__builtin_fma(-b, q, a), r, q);
+}
+
+__device__ __forceinline__ double fastRsqrt(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = __builtin_fma(-(x * y), y, 1.0);
+  return __builtin_fma(y * e, __builtin_fma(0.375, e, 0.5), y);
+}
+
+__device__ __forceinline__ double fastSqrt(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  const double r = __builtin_fma(-h, g, 0.5);
+  g = __builtin_fma(g, r, g);
+  h = __builtin_fma(h, r, h);
+  g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+  return x == 0. ? x : g;
 }
 
 }  // namespace grim

@@ -84,7 +84,8 @@ __global__ __launch_bounds__(kDefaultBlock) void newtonGlobalUpdate(DevParams pr
   int evals = 0;
   ZoneScale zs{};
   EmhdWeights ew;
-  newtonUpdate<L, MODE_FD>(P, R, l2buf[z], G, c, prm, batchDt(b), zs, ew, Rt, evals);
+  FusedPrimal f;
+  newtonUpdate<L, MODE_FD>(P, R, l2buf[z], G, c, prm, batchDt(b), zs, ew, f, Rt, evals);
 #pragma unroll
   for (int v = 0; v < L::NF; v++) b.prim[v * n + z] = P[v];
   evalsBuf[z] += evals;
@@ -394,7 +395,6 @@ int batchedNewton(const grim_params* p, const grim_zone_batch* b, const grim_new
   cfg.block = o.block_size ? o.block_size : kDefaultBlock;
   cfg.compaction = o.compaction == 1 || escalate;
   cfg.workgroupSplit = o.compaction == 2 && !escalate;
-  cfg.escalate = escalate;
   cfg.budget1 = o.phase1_iters ? o.phase1_iters : 2;
   cfg.group = o.phase2_group ? o.phase2_group : 1;
   // persistent phase 2: 8 wavefronts per compute unit

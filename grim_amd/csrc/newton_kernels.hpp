@@ -21,6 +21,7 @@
 
 #include "analytic.hpp"
 #include "fold.hpp"
+#include "fused.hpp"
 #include "grim_hip.h"
 #include "zone_physics.hpp"
 
@@ -37,20 +38,16 @@ __device__ __forceinline__ double batchDt(const grim_zone_batch& b) {
 // Jacobian / precision modes of the per-zone Newton kernel.
 //  MODE_FD:          grim's residual and FD Jacobian, FP64 LU (reference path)
 //  MODE_ANALYTIC64:  grim's residual, analytic Jacobian and LU in FP64
-//  MODE_MIXED:       FP64 residual (reciprocal form) and update; analytic
-//                    Jacobian and equilibrated LU in FP32
+//  MODE_MIXED:       fused FP64 residual; the analytic Newton step by
+//                    elimination (newtonStep, fused.hpp), in FP64
 //  MODE_FD_FAST:     grim's FD Jacobian rule on the reciprocal-form FP64
 //                    residual, one reciprocal per FD column, FP64 LU (the
 //                    fastest FD-FP64 variant, for a like-for-like comparison)
-//  MODE_ANALYTIC64F: the mixed path's FP64 escalation: MODE_MIXED's residual
-//                    with the analytic Jacobian and LU in FP64 (phase 2 of
-//                    GRIM_LU_FP32_FP64, compiled in the fused unit)
-enum { MODE_FD = 0, MODE_ANALYTIC64 = 1, MODE_MIXED = 2, MODE_FD_FAST = 3, MODE_ANALYTIC64F = 4 };
+enum { MODE_FD = 0, MODE_ANALYTIC64 = 1, MODE_MIXED = 2, MODE_FD_FAST = 3 };
 
 template <int MODE>
 struct ModeTraits {
-  static constexpr bool fastResidual = (MODE == MODE_MIXED || MODE == MODE_FD_FAST || MODE == MODE_ANALYTIC64F);
-  static constexpr bool analytic = (MODE == MODE_ANALYTIC64 || MODE == MODE_MIXED || MODE == MODE_ANALYTIC64F);
+  static constexpr bool fused = (MODE == MODE_MIXED || MODE == MODE_FD_FAST);
 };
 
 // The EMHD mixed solve keeps each zone's metric (16 doubles) and EMHD
@@ -70,23 +67,14 @@ __device__ __forceinline__ void slotFence() {
   if constexpr (kLdsState<L, MODE>) asm volatile("" ::: "memory");
 }
 
-// Per-zone quantities of the residual formed once per zone.
-struct ZoneScale {
-  double invAlpha;  // 1/alpha
-  double scale;     // mask/dt
-  double invDt;     // 1/dt
-};
-
 template <class L, int MODE>
 __device__ __forceinline__ void evalResidual(const double* P, const ZoneGeom& G,
                                              const ZoneConst<L>& c, const DevParams& prm,
                                              double dt, const ZoneScale& zs, const EmhdWeights& ew,
-                                             double* R) {
+                                             double* R, FusedPrimal& f) {
   slotFence<L, MODE>();
-  if constexpr (ModeTraits<MODE>::fastResidual && !L::EMHD)
-    residualFastIdeal<L>(P, G, c, prm, zs.invAlpha, zs.scale, R);
-  else if constexpr (ModeTraits<MODE>::fastResidual)
-    residualFastEmhd<L>(P, G, c, prm, ew, zs.invDt, R);
+  if constexpr (ModeTraits<MODE>::fused)
+    residualFused<L>(P, G, c, prm, zs, ew, R, f);
   else
     residual<L>(P, G, c, prm, dt, R);
 }
@@ -165,14 +153,15 @@ __device__ __forceinline__ void fdJacobianWide(const double* P, const double* R,
 
 // One Newton update after the convergence test (solve.cpp:80-198): Jacobian,
 // LU solve of J d = -R, quadratic backtracking line search, P += lambda d.
-// Returns true when the last evaluated trial was accepted; Rt then holds the
-// residual at the new P (bit-identical to a fresh evaluation, since the new P
-// is computed by the same expression as the trial).
+// Returns true when the last evaluated trial was accepted; Rt (and f, the
+// primal of the fused modes) then holds the residual at the new P
+// (bit-identical to a fresh evaluation, since the new P is computed by the
+// same expression as the trial).
 template <class L, int MODE, bool WIDE = false>
 __device__ __forceinline__ bool newtonUpdate(double* P, const double* R, double l2,
                                              const ZoneGeom& G, const ZoneConst<L>& c,
                                              const DevParams& prm, double dt, const ZoneScale& zs,
-                                             const EmhdWeights& ew, double* Rt, int& evals) {
+                                             const EmhdWeights& ew, FusedPrimal& f, double* Rt, int& evals) {
   double d[L::NF];
   if constexpr (MODE == MODE_FD) {
     double A[L::NF][L::NF];
@@ -191,21 +180,15 @@ __device__ __forceinline__ bool newtonUpdate(double* P, const double* R, double 
 #pragma unroll
     for (int v = 0; v < L::NF; v++) d[v] = -R[v];
     luSolve<double, L::NF>(A, d);
-  } else if constexpr (MODE == MODE_ANALYTIC64 || MODE == MODE_ANALYTIC64F) {
+  } else if constexpr (MODE == MODE_ANALYTIC64) {
     double A[L::NF][L::NF];
     analyticJacobian<double, L>(P, G, prm, c.mask / dt, c, ew, dt, A);
 #pragma unroll
     for (int v = 0; v < L::NF; v++) d[v] = -R[v];
     luSolve<double, L::NF>(A, d);
   } else {
-    float A[L::NF][L::NF], df[L::NF];
     slotFence<L, MODE>();
-    analyticJacobian<float, L>(P, G, prm, c.mask / dt, c, ew, dt, A);
-#pragma unroll
-    for (int v = 0; v < L::NF; v++) df[v] = (float)(-R[v]);
-    equilibratedSolve<float, L::NF>(A, df, P);
-#pragma unroll
-    for (int v = 0; v < L::NF; v++) d[v] = (double)df[v];
+    newtonStep<L>(P, R, G, c, prm, zs, ew, f, d);
   }
 
   const double f0 = 0.5 * l2;
@@ -219,7 +202,7 @@ __device__ __forceinline__ bool newtonUpdate(double* P, const double* R, double 
   for (int ls = 0; ls < prm.maxLS; ls++) {
 #pragma unroll
     for (int v = 0; v < L::NF; v++) Pt[v] = P[v] + lambda * d[v];
-    evalResidual<L, MODE>(Pt, G, c, prm, dt, zs, ew, Rt);
+    evalResidual<L, MODE>(Pt, G, c, prm, dt, zs, ew, Rt, f);
     evals += 1;
     const double f1 = 0.5 * sumSq<L::NF>(Rt);
     if constexpr (MODE == MODE_FD) {
@@ -230,9 +213,9 @@ __device__ __forceinline__ bool newtonUpdate(double* P, const double* R, double 
         break;
       }
     } else {
-      // this build's solvers reject a non-finite trial and halve the step
-      // (an FP32 Jacobian of a near-singular zone can overshoot into
-      // states where the residual overflows)
+      // this build's solvers reject a non-finite trial and halve the step (a
+      // near-singular zone can overshoot into states where the residual
+      // overflows)
       finiteTrial = isfinite(f1);
       if (f1 <= f0 * (1. - 1e-4 * lambda) + prm.lsFloor) {
         accepted = true;
@@ -301,21 +284,20 @@ __device__ __forceinline__ bool solveZone(const DevParams& prm, const grim_zone_
   ZoneGeom G;
   loadBatchGeom(b, z, G);
   ZoneConst<L> c;
-  loadZoneConst<L, !FOLDED>(b, prm, G, z, c);
-  if constexpr (FOLDED) {
+  ZoneScale zs;
+  EmhdWeights ew;
+  if constexpr (!ModeTraits<MODE>::fused) loadZoneConst<L, !FOLDED>(b, prm, G, z, c);
+  if constexpr (ModeTraits<MODE>::fused || FOLDED) {
 #pragma unroll
-    for (int v = 0; v < L::NF; v++) c.rhs[v] = foldRhs[v];
+    for (int v = 0; v < L::NF; v++) c.rhs[v] = FOLDED ? foldRhs[v] : b.rhs[v * n + z];
     c.mask = maskZ;
   }
-  ZoneScale zs;
-  if constexpr (ModeTraits<MODE>::fastResidual) {
-    zs.invAlpha = 1. / G.alpha;
-    zs.scale = c.mask / dt;
-    zs.invDt = 1. / dt;
-  }
-  EmhdWeights ew;
-  if constexpr (L::EMHD && (ModeTraits<MODE>::analytic || ModeTraits<MODE>::fastResidual))
+  if constexpr (ModeTraits<MODE>::fused) {
+    zoneScale(G, maskZ, dt, zs);
+    if constexpr (L::EMHD) fusedEmhdConstants<L>(b, prm, G, z, zs.invDt, c, ew);
+  } else if constexpr (MODE == MODE_ANALYTIC64 && L::EMHD) {
     emhdWeights<L>(G, c, prm, dt, ew);
+  }
   if constexpr (kLdsState<L, MODE>) {
     static_assert(sizeof(ZoneGeom) <= kGeomSlot * sizeof(double) &&
                   sizeof(EmhdWeights) <= kWeightSlot * sizeof(double), "LDS slot sizes");
@@ -348,6 +330,7 @@ __device__ __forceinline__ bool solveZoneCore(const DevParams& prm, const grim_z
     P[v] = v < L::NF ? start[v * n + z] : (foldB ? foldB[v - L::NF] : b.prim[v * n + z]);
 
   double R[L::NF];
+  FusedPrimal f;
   bool haveR = false;
   bool converged = false;
   int iters = 0, evals = 0;
@@ -360,7 +343,7 @@ __device__ __forceinline__ bool solveZoneCore(const DevParams& prm, const grim_z
     P[RHO] = p0;
     P[UU] = p1;
     if (!haveR) {
-      evalResidual<L, MODE>(P, G, c, prm, dt, zs, ew, R);
+      evalResidual<L, MODE>(P, G, c, prm, dt, zs, ew, R, f);
       evals++;
     }
     l2 = sumSq<L::NF>(R);
@@ -369,7 +352,7 @@ __device__ __forceinline__ bool solveZoneCore(const DevParams& prm, const grim_z
       break;
     }
     double Rt[L::NF];
-    haveR = newtonUpdate<L, MODE, WIDE>(P, R, l2, G, c, prm, dt, zs, ew, Rt, evals);
+    haveR = newtonUpdate<L, MODE, WIDE>(P, R, l2, G, c, prm, dt, zs, ew, f, Rt, evals);
     iters++;
     if (haveR) {
 #pragma unroll
@@ -378,7 +361,7 @@ __device__ __forceinline__ bool solveZoneCore(const DevParams& prm, const grim_z
   }
   if (!converged) {
     if (!haveR) {
-      evalResidual<L, MODE>(P, G, c, prm, dt, zs, ew, R);
+      evalResidual<L, MODE>(P, G, c, prm, dt, zs, ew, R, f);
       if (!lastPhase) evals++;
     }
     l2 = sumSq<L::NF>(R);
@@ -636,7 +619,8 @@ __device__ __forceinline__ void fdJacobianFast(const double* P, const double* R,
     const bool small = fabs(P[row]) < .5 * eps;
     Pp[row] = small ? P[row] + eps : P[row] + eps * P[row];
     double Rp[L::NF];
-    evalResidual<L, MODE>(Pp, G, c, prm, dt, zs, ew, Rp);
+    FusedPrimal f;
+    evalResidual<L, MODE>(Pp, G, c, prm, dt, zs, ew, Rp, f);
     const double inv = 1. / (Pp[row] - P[row]);
 #pragma unroll
     for (int col = 0; col < L::NF; col++) A[col][row] = (Rp[col] - R[col]) * inv;
@@ -686,7 +670,6 @@ struct LaunchCfg {
   int budget1;               // phase-1 update budget
   int group;                 // phase-2 grab: chunks of 64 list entries per atomic (1..kMaxGroup)
   int persistentWaves;       // phase-2 grid, in wavefronts
-  bool escalate;             // mixed path: phase 2 in FP64 (GRIM_LU_FP32_FP64)
   CompactionWorkspace ws;    // masks, prefix sums, work list, counters
 };
 
@@ -696,11 +679,10 @@ constexpr size_t ldsBytes(int block) {
   return kLdsState<L, MODE> ? kLdsStateBytes * (size_t)block : 0;
 }
 
-// Enqueue the per-zone solve of mode MODE on stream s (phase 2 of the
-// compacting solve in MODE2).
+// Enqueue the per-zone solve of mode MODE on stream s.
 // fold: a grid stage's fold runs inside phase 1 (newtonPhase1Fold; the
 // caller has checked that the solve compacts, see foldFusable).
-template <class L, int MODE, int MODE2 = MODE>
+template <class L, int MODE>
 void launchSolve(const DevParams& prm, const grim_zone_batch& b, const grim_newton_stats& st,
                  const LaunchCfg& cfg, hipStream_t s, const FoldArgs* fold = nullptr) {
   const unsigned grid = (unsigned)((b.n + cfg.block - 1) / cfg.block);
@@ -718,7 +700,6 @@ void launchSolve(const DevParams& prm, const grim_zone_batch& b, const grim_newt
       newtonPerZone<L, MODE><<<grid, cfg.block, ldsBytes<L, MODE>(cfg.block), s>>>(prm, b, st);
     return;
   }
-  static_assert(MODE2 == MODE || (MODE == MODE_MIXED && MODE2 == MODE_ANALYTIC64F), "phase-2 mode");
   const CompactionWorkspace& w = cfg.ws;
   if constexpr (MODE == MODE_MIXED) {
     if (fold)
@@ -737,7 +718,7 @@ void launchSolve(const DevParams& prm, const grim_zone_batch& b, const grim_newt
   scatterListKernel<<<(unsigned)nScan, kScanBlock, 0, s>>>(nMasks, w.masks, w.maskOff, w.blockSum, w.list);
   const int64_t waves = std::min<int64_t>(cfg.persistentWaves, nMasks);
   const unsigned grid2 = (unsigned)((waves * 64 + cfg.block - 1) / cfg.block);
-  newtonPhase2<L, MODE2><<<grid2, cfg.block, ldsBytes<L, MODE2>(cfg.block), s>>>(
+  newtonPhase2<L, MODE><<<grid2, cfg.block, ldsBytes<L, MODE>(cfg.block), s>>>(
       prm, b, st, prm.maxIter - cfg.budget1, w.list, w.ctrl, cfg.group);
 }
 

@@ -411,23 +411,19 @@ __device__ __forceinline__ double sumSq(const double* R) {
 // eliminated by the same operations wherever it sits, so the solution is
 // bit-identical to the search-then-swap order (exact ties aside).  Every
 // access stays at a compile-time index: a swap with a computed row index
-// would force the matrix out of registers into scratch memory.  PIVOT false
-// factorises in the given row order (the mixed path's equilibrated FP32
-// systems).
+// would force the matrix out of registers into scratch memory. 
 
-// 1/x: FP64 correctly rounded; FP32 the hardware reciprocal (within one ulp;
-// the FP32 factorisation is an approximate solve refined by the FP64 Newton
-// updates around it).
+// 1/x: FP64 correctly rounded; FP32 the hardware reciprocal (within one ulp).
 __device__ __forceinline__ double lowRecip(double x) { return 1. / x; }
 __device__ __forceinline__ float lowRecip(float x) { return __builtin_amdgcn_rcpf(x); }
 
-template <class Real, int N, bool PIVOT = true>
+template <class Real, int N>
 __device__ __forceinline__ void luSolve(Real (&A)[N][N], Real (&b)[N]) {
   Real rinv[N];
 #pragma unroll
   for (int k = 0; k < N; k++) {
 #pragma unroll
-    for (int i = k + 1; i < N && PIVOT; i++) {
+    for (int i = k + 1; i < N; i++) {
       const bool swap = fabs(A[i][k]) > fabs(A[k][k]);
 #pragma unroll
       for (int j = k; j < N; j++) {

@@ -116,10 +116,13 @@ typedef struct grim_zone_batch {
 typedef enum grim_jacobian_kind { GRIM_JAC_FD = 0, GRIM_JAC_ANALYTIC = 1 } grim_jacobian_kind;
 typedef enum grim_lu_precision {
   GRIM_LU_FP64 = 0,
-  GRIM_LU_FP32 = 1,
-  GRIM_LU_FP32_FP64 = 2 /* analytic Jacobian only: FP32 Jacobian and LU for the
-                           first phase1_iters updates of each zone, FP64 for
-                           the rest (always run as the compacting solve) */
+  GRIM_LU_FP32 = 1, /* the fused analytic solve: the caller admits FP32 for the
+                       Jacobian and its factorisation.  The solve eliminates
+                       the Newton system by its structure in FP64, which is
+                       cheaper than assembling and factorising an FP32 matrix */
+  GRIM_LU_FP32_FP64 = 2 /* analytic Jacobian only: the same fused solve, always
+                           run as the compacting solve (FP32 admitted for the
+                           first phase1_iters updates of a zone only) */
 } grim_lu_precision;
 typedef enum grim_semantics {
   GRIM_NEWTON_PER_ZONE = 0, /* each zone stops at its own convergence */

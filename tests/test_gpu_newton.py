@@ -296,6 +296,49 @@ def test_analytic_newton_converges_to_fd_solution(capi, torch_cuda, oracle, mode
         assert np.median(rel_star[ok]) < 1e-9
 
 
+@pytest.mark.parametrize("n", [1, 63, 257, 4099])
+@pytest.mark.parametrize("cond,visc,high", [(0, 0, 1), (1, 0, 1), (0, 1, 1), (1, 1, 1), (1, 1, 0)])
+def test_eliminated_newton_step_solves_the_dense_system(capi, torch_cuda, cond, visc, high, n):
+    """One update of the fused path (the step by elimination) against the
+    dense analytic Jacobian: J d = -R row by row, for zones that took the
+    full step.  Bound: the backward error of the elimination, 1e-9 of the
+    row's terms (a few hundred roundings times the growth of a 3x3
+    elimination), d's own rounding in P + d (eps |P_j| times |J_ij|), and
+    2e-11 for R itself: the rows are scaled to |rhs| <= 1, and the fused
+    residual's metric identities (u_0 = -alpha gamma + g_0j utilde^j) hold to
+    the rounding of the batch's metric and its inverse, eps times a condition
+    number of up to 1e5."""
+    torch = torch_cuda
+    p = capi.default_params(True)
+    p.conduction, p.viscosity = cond, visc
+    p.highOrderTermsConduction = p.highOrderTermsViscosity = high
+    p.maxNonLinearIter = 1
+    emhd = cond or visc
+    p.closure = capi.CLOSURE_PER_ZONE if emhd else capi.CLOSURE_LINEAR_MODES
+    b = capi.generate_kerr_schild_batch(p, n, SEED + n)
+    rhs = torch.empty((p.nf, n), dtype=torch.float64, device="cuda")
+    mask = torch.empty(n, dtype=torch.float64, device="cuda")
+    capi.known_root_rhs(p, capi.make_batch(b["prim_star"], b["geom"], rhs, b["prim_old"], None, b["closure"]), rhs, mask)
+    prim = b["guess"].clone()
+    batch = capi.make_batch(prim, b["geom"], rhs, b["prim_old"], None, b["closure"], residual_mask=mask)
+    J = torch.empty((p.nf * p.nf, n), dtype=torch.float64, device="cuda")
+    R = torch.empty((p.nf, n), dtype=torch.float64, device="cuda")
+    capi.jacobian(p, batch, capi.JAC_ANALYTIC, J)
+    capi.residual(p, batch, R)
+    ev = torch.zeros(n, dtype=torch.int32, device="cuda")
+    capi.batched_newton(p, batch, capi.JAC_ANALYTIC, capi.LU_FP32, residual_evals=ev)
+    torch.cuda.synchronize()
+    J, R, P0, P1, ev = host(J).reshape(p.nf, p.nf, n), host(R), host(b["guess"])[: p.nf], host(prim)[: p.nf], host(ev)
+    full = ev == 2  # the first residual and one accepted trial
+    assert full.mean() > 0.5 or n == 1
+    d = P1 - P0
+    err = np.abs(np.einsum("ijz,jz->iz", J, d) + R)
+    bound = np.einsum("ijz,jz->iz", np.abs(J), 1e-9 * np.abs(d) + 2.3e-16 * np.abs(P0)) + 1e-9 * np.abs(R) + 2e-11
+    ratio = (err / bound)[:, full]
+    print(f"step: {int(full.sum())} of {n} zones, worst row {ratio.max() if full.any() else 0:.2e} of the bound")
+    assert (ratio <= 1.).all()
+
+
 # ------------------------------------------------ compaction, autotune, graphs
 @pytest.mark.parametrize("case", [("fd", False, 1), ("fd", True, 2), ("mixed", False, 1), ("mixed", False, 2),
                                   ("fd_fused", True, 3)])
