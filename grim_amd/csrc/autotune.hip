@@ -3,9 +3,8 @@
 // Times each candidate launch configuration on the caller's batch (on a
 // scratch copy of the primitives, restored before every run) with HIP
 // events and keeps the fastest.  Candidates: workgroup size 64/128/256;
-// one pass, or the two-phase compacting solve with a phase-1 budget of
-// 1-3 Newton updates and 2, 4 or 8 phase-1 wavefronts per phase-2
-// wavefront.  The timing is the median of three runs.
+// one pass, or either compacting solve with a phase-1 budget of 1-3 Newton
+// updates.  The timing is the median of three runs.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -46,14 +45,10 @@ extern "C" int grim_autotune_newton(const grim_params* p, const grim_zone_batch*
       o.phase1_iters = k1;
       o.phase2_group = 0;
       cands.push_back(o);
-      for (int g : {2, 4, 8}) {
-        o.compaction = 1;
-        o.phase1_iters = k1;
-        o.phase2_group = g;
-        o.workspace = ws;
-        o.workspace_bytes = wsBytes;
-        cands.push_back(o);
-      }
+      o.compaction = 1;
+      o.workspace = ws;
+      o.workspace_bytes = wsBytes;
+      cands.push_back(o);
     }
   }
   grim_zone_batch bb = *b;

@@ -396,8 +396,7 @@ int batchedNewton(const grim_params* p, const grim_zone_batch* b, const grim_new
   cfg.compaction = o.compaction == 1 || escalate;
   cfg.workgroupSplit = o.compaction == 2 && !escalate;
   cfg.budget1 = o.phase1_iters ? o.phase1_iters : 2;
-  cfg.group = o.phase2_group ? o.phase2_group : 1;
-  // persistent phase 2: 8 wavefronts per compute unit
+  // phase 2: 8 wavefronts per compute unit
   cfg.persistentWaves = 8 * deviceCUs();
   cfg.ws = CompactionWorkspace{};
   void* owned = nullptr;
@@ -542,7 +541,7 @@ int grim_batch_linear_solve(int64_t n, int nvar, const double* A, const double* 
 }
 
 int64_t grim_newton_workspace_bytes(int64_t n) {
-  // phase-1 masks, their prefix sums, the work list and two counters
+  // per phase-1 wavefront, the zones handed over and their update count
   return n < 0 ? 0 : compactionBytes(n);
 }
 

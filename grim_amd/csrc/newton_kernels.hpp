@@ -28,7 +28,7 @@
 namespace grim {
 
 constexpr int kDefaultBlock = 256;
-constexpr int kMaxGroup = 8;  // phase-2 grab, in chunks of 64 list entries, at most
+constexpr int kMaxGroup = 8;  // largest grim_newton_opts.phase2_group taken
 
 // dt' of the batch: from device memory when the caller computed it there.
 __device__ __forceinline__ double batchDt(const grim_zone_batch& b) {
@@ -238,27 +238,29 @@ __device__ __forceinline__ bool newtonUpdate(double* P, const double* R, double 
 }
 
 // Newton iterations of one zone, from its current primitives, for at most
-// `budget` updates (solve.cpp:10-200 read per zone: the zone stops when its
+// `limit` updates (solve.cpp:10-200 read per zone: the zone stops when its
 // own sum R^2 <= atol).  Writes the primitives back; stats are stored, or
-// added to the earlier phase's when `accumulate`.  Returns true when the
-// zone ran out of budget unconverged (a later phase may continue it: every
+// added to the earlier phase's when `accumulate`.  Once `budget` updates are
+// done, a wavefront left with fewer than `keep` unconverged zones stops too:
+// returns true then, with the updates done in `done` (the same for every
+// lane that returns true), and a later phase continues the zone -- every
 // iteration is a function of P alone, so stopping and resuming changes no
-// result).  WIDE: the zone's kWide lanes run it together; only the first
+// result.  WIDE: the zone's kWide lanes run it together; only the first
 // writes.
 template <class L, int MODE, bool WIDE>
 __device__ __forceinline__ bool solveZoneCore(const DevParams& prm, const grim_zone_batch& b,
-                                              const grim_newton_stats& st, int64_t z, int budget,
-                                              bool accumulate, bool lastPhase, double dt, const ZoneGeom& G,
+                                              const grim_newton_stats& st, int64_t z, int budget, int limit,
+                                              int keep, bool accumulate, double dt, const ZoneGeom& G,
                                               const ZoneConst<L>& c, const ZoneScale& zs, const EmhdWeights& ew,
-                                              const double* start, const double* foldB);
+                                              const double* start, const double* foldB, int& done);
 
 // FOLDED: the zone's right-hand side, field rows and residual mask come from
 // the caller's registers (foldRhs, foldB, foldMask: the stage fold computed
 // in the same kernel) instead of the batch's planes.
 template <class L, int MODE, bool WIDE = false, bool FOLDED = false>
 __device__ __forceinline__ bool solveZone(const DevParams& prm, const grim_zone_batch& b,
-                                          const grim_newton_stats& st, int64_t z, int budget,
-                                          bool accumulate, bool lastPhase, const double* foldRhs = nullptr,
+                                          const grim_newton_stats& st, int64_t z, int budget, int limit,
+                                          int keep, bool accumulate, int& done, const double* foldRhs = nullptr,
                                           const double* foldB = nullptr, double foldMask = 0.) {
   const int64_t n = b.n;
   const bool lead = !WIDE || (threadIdx.x % kWide) == 0;
@@ -308,20 +310,20 @@ __device__ __forceinline__ bool solveZone(const DevParams& prm, const grim_zone_
         reinterpret_cast<EmhdWeights*>(zoneSlots + (size_t)kGeomSlot * blockDim.x + (size_t)kWeightSlot * threadIdx.x);
     *gs = G;
     *ws = ew;
-    return solveZoneCore<L, MODE, WIDE>(prm, b, st, z, budget, accumulate, lastPhase, dt, *gs, c, zs, *ws, start,
-                                        FOLDED ? foldB : nullptr);
+    return solveZoneCore<L, MODE, WIDE>(prm, b, st, z, budget, limit, keep, accumulate, dt, *gs, c, zs, *ws, start,
+                                        FOLDED ? foldB : nullptr, done);
   } else {
-    return solveZoneCore<L, MODE, WIDE>(prm, b, st, z, budget, accumulate, lastPhase, dt, G, c, zs, ew, start,
-                                        FOLDED ? foldB : nullptr);
+    return solveZoneCore<L, MODE, WIDE>(prm, b, st, z, budget, limit, keep, accumulate, dt, G, c, zs, ew, start,
+                                        FOLDED ? foldB : nullptr, done);
   }
 }
 
 template <class L, int MODE, bool WIDE>
 __device__ __forceinline__ bool solveZoneCore(const DevParams& prm, const grim_zone_batch& b,
-                                              const grim_newton_stats& st, int64_t z, int budget,
-                                              bool accumulate, bool lastPhase, double dt, const ZoneGeom& G,
+                                              const grim_newton_stats& st, int64_t z, int budget, int limit,
+                                              int keep, bool accumulate, double dt, const ZoneGeom& G,
                                               const ZoneConst<L>& c, const ZoneScale& zs, const EmhdWeights& ew,
-                                              const double* start, const double* foldB) {
+                                              const double* start, const double* foldB, int& done) {
   const int64_t n = b.n;
   const bool lead = !WIDE || (threadIdx.x % kWide) == 0;
   double P[L::DOF];
@@ -332,10 +334,10 @@ __device__ __forceinline__ bool solveZoneCore(const DevParams& prm, const grim_z
   double R[L::NF];
   FusedPrimal f;
   bool haveR = false;
-  bool converged = false;
+  bool converged = false, handOver = false;
   int iters = 0, evals = 0;
   double l2 = 0.;
-  for (int it = 0; it < budget; it++) {
+  while (iters < limit) {
     // floors at the top of every iteration (solve.cpp:17-18)
     const double p0 = smax(P[RHO], prm.rhoFloor);
     const double p1 = smax(P[UU], prm.uFloor);
@@ -351,6 +353,10 @@ __device__ __forceinline__ bool solveZoneCore(const DevParams& prm, const grim_z
       converged = true;
       break;
     }
+    if (iters >= budget && __popcll(__ballot(1)) < keep) {
+      handOver = true;
+      break;
+    }
     double Rt[L::NF];
     haveR = newtonUpdate<L, MODE, WIDE>(P, R, l2, G, c, prm, dt, zs, ew, f, Rt, evals);
     iters++;
@@ -359,27 +365,19 @@ __device__ __forceinline__ bool solveZoneCore(const DevParams& prm, const grim_z
       for (int v = 0; v < L::NF; v++) R[v] = Rt[v];
     }
   }
-  if (!converged) {
-    if (!haveR) {
-      evalResidual<L, MODE>(P, G, c, prm, dt, zs, ew, R, f);
-      if (!lastPhase) evals++;
-    }
+  if (!converged && !handOver) {
+    // out of updates: the statistics take the residual where the zone ended
+    if (!haveR) evalResidual<L, MODE>(P, G, c, prm, dt, zs, ew, R, f);
     l2 = sumSq<L::NF>(R);
-    if (!lastPhase && !(l2 > prm.atol)) {
-      // the one-pass solve would floor P at the top of its next iteration
-      // and then stop: do the same here
-      P[RHO] = smax(P[RHO], prm.rhoFloor);
-      P[UU] = smax(P[UU], prm.uFloor);
-      converged = true;
-    }
   }
-  if (!lead) return !converged && !lastPhase;
+  done = iters;
+  if (!lead) return handOver;
 #pragma unroll
   for (int v = 0; v < L::NF; v++) b.prim[v * n + z] = P[v];
   if (st.iterations) st.iterations[z] = (accumulate ? st.iterations[z] : 0) + iters;
   if (st.residual_evals) st.residual_evals[z] = (accumulate ? st.residual_evals[z] : 0) + evals;
   if (st.final_l2) st.final_l2[z] = l2;
-  return !converged && !lastPhase;
+  return handOver;
 }
 
 // Per-zone semantics, one pass: each thread iterates its own zone until
@@ -393,7 +391,8 @@ __global__ __launch_bounds__(kDefaultBlock) __attribute__((amdgpu_waves_per_eu(2
     DevParams prm, grim_zone_batch b, grim_newton_stats st) {
   const int64_t z = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (z >= b.n) return;
-  solveZone<L, MODE>(prm, b, st, z, prm.maxIter, false, true);
+  int done;
+  solveZone<L, MODE>(prm, b, st, z, prm.maxIter, prm.maxIter, 0, false, done);
 }
 
 // One-pass per-zone solve with the stragglers gathered inside the workgroup:
@@ -417,7 +416,8 @@ __global__ __launch_bounds__(kDefaultBlock) __attribute__((amdgpu_waves_per_eu(2
   __shared__ int waveCount[kDefaultBlock / 64];
   const int64_t z = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   bool more = false;
-  if (z < b.n) more = solveZone<L, MODE>(prm, b, st, z, budget1, false, false);
+  int done;
+  if (z < b.n) more = solveZone<L, MODE>(prm, b, st, z, budget1, prm.maxIter, 65, false, done);
   const unsigned long long ballot = __ballot(more);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (lane == 0) waveCount[wave] = __popcll(ballot);
@@ -430,7 +430,7 @@ __global__ __launch_bounds__(kDefaultBlock) __attribute__((amdgpu_waves_per_eu(2
   if (more) list[base + __popcll(ballot & ((1ull << lane) - 1ull))] = (int)z;
   __syncthreads();
   if ((int)threadIdx.x < total)
-    solveZone<L, MODE>(prm, b, st, (int64_t)list[threadIdx.x], prm.maxIter - budget1, true, true);
+    solveZone<L, MODE>(prm, b, st, (int64_t)list[threadIdx.x], prm.maxIter, prm.maxIter - budget1, 0, true, done);
 }
 
 // The one-pass FD solve of a small batch, kWide lanes per zone (every lane
@@ -440,22 +440,48 @@ __global__ __launch_bounds__(kDefaultBlock) void newtonPerZoneWide(DevParams prm
                                                                   grim_newton_stats st) {
   const int64_t z = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWide;
   if (z >= b.n) return;
-  solveZone<L, MODE_FD, true>(prm, b, st, z, prm.maxIter, false, true);
+  int done;
+  solveZone<L, MODE_FD, true>(prm, b, st, z, prm.maxIter, prm.maxIter, 0, false, done);
 }
 
-// Compacting solve, phase 1: at most `budget1` updates per zone.  Each
-// wavefront stores the 64-bit ballot of its lanes left unconverged (no
-// atomics: a single global counter serialises 65536 wavefronts).
+// The compacting solve.  Phase 1 gives every zone `budget1` updates, and goes
+// on while a wavefront holds at least kKeepLanes unconverged zones; what is
+// left it hands over as one 64-bit mask of lanes and one update count per
+// wavefront.  Phase 2's wavefronts gather those zones, 64 at a time.
+//
+// Handing a zone over costs its planes again, 64-byte sectors of which it
+// uses one entry (about 45 planes of an EMHD zone: 2.9 KB, the share of
+// 1,300 cycles of a SIMD at the memory's rate), so it pays only where the
+// update a wavefront would repeat for the zone's sake is dearer: about 2,800
+// cycles for the fused step (three lanes), 10,000 for the dense analytic one
+// and 20,000 and more for finite differences.  With every straggler handed
+// over after two updates, a fifth of the 700,001-zone EMHD batch, phase 2
+// took 75 us and the list 15 us beside phase 1's 83; now 100 and 5 us.
+template <int MODE>
+constexpr int kKeepLanes = MODE == MODE_MIXED ? 3 : (MODE == MODE_ANALYTIC64 ? 6 : 12);
+
+// Lane 0 of a wavefront holding at least one zone stores what it hands over;
+// wavefronts wholly past the end of the batch own no entry.
+__device__ __forceinline__ void storeHandOver(bool more, int done, int64_t z, int64_t n,
+                                              unsigned long long* __restrict__ masks, int* __restrict__ updates) {
+  const unsigned long long ballot = __ballot(more);
+  const int first = ballot ? __ffsll((long long)ballot) - 1 : 0;
+  const int count = __shfl(done, first, 64);
+  if ((threadIdx.x & 63) == 0 && z < n) {
+    masks[z >> 6] = ballot;
+    updates[z >> 6] = count;
+  }
+}
+
 template <class L, int MODE>
 __global__ __launch_bounds__(kDefaultBlock) __attribute__((amdgpu_waves_per_eu(2))) void newtonPhase1(
-    DevParams prm, grim_zone_batch b, grim_newton_stats st, int budget1, unsigned long long* __restrict__ masks) {
+    DevParams prm, grim_zone_batch b, grim_newton_stats st, int budget1, unsigned long long* __restrict__ masks,
+    int* __restrict__ updates) {
   const int64_t z = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   bool more = false;
-  if (z < b.n) more = solveZone<L, MODE>(prm, b, st, z, budget1, false, false);
-  const unsigned long long ballot = __ballot(more);
-  // lane 0 of a wavefront holding at least one zone (z < n) owns mask z/64;
-  // wavefronts wholly past the end of the batch own none
-  if ((threadIdx.x & 63) == 0 && z < b.n) masks[z >> 6] = ballot;
+  int done = 0;
+  if (z < b.n) more = solveZone<L, MODE>(prm, b, st, z, budget1, prm.maxIter, kKeepLanes<MODE>, false, done);
+  storeHandOver(more, done, z, b.n, masks, updates);
 }
 
 // Phase 1 of a grid stage's compacting solve with the stage fold in front of
@@ -468,9 +494,10 @@ __global__ __launch_bounds__(kDefaultBlock) __attribute__((amdgpu_waves_per_eu(2
 template <class L, int MODE, int DIM>
 __global__ __launch_bounds__(kDefaultBlock) __attribute__((amdgpu_waves_per_eu(2))) void newtonPhase1Fold(
     DevParams prm, grim_zone_batch b, grim_newton_stats st, int budget1, unsigned long long* __restrict__ masks,
-    FoldArgs f) {
+    int* __restrict__ updates, FoldArgs f) {
   const int64_t z = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   bool more = false;
+  int done = 0;
   if (z < b.n) {
     const int64_t n = b.n;
     int i, j, k;
@@ -497,112 +524,69 @@ __global__ __launch_bounds__(kDefaultBlock) __attribute__((amdgpu_waves_per_eu(2
 #pragma unroll
       for (int c = 0; c < 3; c++) b.prim[(L::NF + c) * n + z] = f.fieldIn[c * n + z];
     }
-    more = solveZone<L, MODE, false, true>(prm, b, st, z, budget1, false, false, rhs, B, mask);
+    more = solveZone<L, MODE, false, true>(prm, b, st, z, budget1, prm.maxIter, kKeepLanes<MODE>, false, done, rhs, B,
+                                           mask);
     if (more)
 #pragma unroll
       for (int v = 0; v < L::NF; v++) f.rhs[v * n + z] = rhs[v];
   }
-  const unsigned long long ballot = __ballot(more);
-  if ((threadIdx.x & 63) == 0 && z < b.n) masks[z >> 6] = ballot;
+  storeHandOver(more, done, z, b.n, masks, updates);
 }
 
-// The work list between the phases.  Phase 1 leaves one 64-bit mask of
-// unconverged lanes per wavefront; an exclusive prefix sum of their
-// popcounts numbers the unconverged zones, which are then scattered, in
-// ascending zone order, into a dense list of zone indices.
-constexpr int kScanBlock = 256;  // masks per scan workgroup
-
-// Prefix sums of the popcounts within each workgroup's kScanBlock masks, and
-// each workgroup's total.
-static __global__ __launch_bounds__(kScanBlock) void scanMasksKernel(int64_t nMasks,
-                                                              const unsigned long long* __restrict__ masks,
-                                                              int* __restrict__ maskOff,
-                                                              int* __restrict__ blockSum) {
-  __shared__ int sh[kScanBlock];
-  const int64_t m = (int64_t)blockIdx.x * kScanBlock + threadIdx.x;
-  const int c = m < nMasks ? __popcll(masks[m]) : 0;
-  sh[threadIdx.x] = c;
-  __syncthreads();
-  // Hillis-Steele inclusive scan in LDS
-  for (int off = 1; off < kScanBlock; off <<= 1) {
-    const int v = (int)threadIdx.x >= off ? sh[threadIdx.x - off] : 0;
-    __syncthreads();
-    sh[threadIdx.x] += v;
-    __syncthreads();
-  }
-  if (m < nMasks) maskOff[m] = sh[threadIdx.x] - c;
-  if (threadIdx.x == kScanBlock - 1) blockSum[blockIdx.x] = sh[threadIdx.x];
-}
-
-// Exclusive prefix over the workgroup totals (one workgroup, in chunks of
-// kScanBlock), the list length into ctrl[0], and the grab counter ctrl[1]
-// cleared for the persistent phase.
-static __global__ __launch_bounds__(kScanBlock) void scanBlocksKernel(int64_t nBlocks, int* __restrict__ blockSum,
-                                                               int* __restrict__ ctrl) {
-  __shared__ int sh[kScanBlock];
-  int carry = 0;
-  for (int64_t base = 0; base < nBlocks; base += kScanBlock) {
-    const int64_t q = base + threadIdx.x;
-    const int c = q < nBlocks ? blockSum[q] : 0;
-    sh[threadIdx.x] = c;
-    __syncthreads();
-    for (int off = 1; off < kScanBlock; off <<= 1) {
-      const int v = (int)threadIdx.x >= off ? sh[threadIdx.x - off] : 0;
-      __syncthreads();
-      sh[threadIdx.x] += v;
-      __syncthreads();
-    }
-    if (q < nBlocks) blockSum[q] = carry + sh[threadIdx.x] - c;
-    const int chunk = sh[kScanBlock - 1];
-    __syncthreads();
-    carry += chunk;
-  }
-  if (threadIdx.x == 0) {
-    ctrl[0] = carry;
-    ctrl[1] = 0;
-  }
-}
-
-// Each mask's unconverged zones into the list at their global rank.
-static __global__ __launch_bounds__(kScanBlock) void scatterListKernel(int64_t nMasks,
-                                                                const unsigned long long* __restrict__ masks,
-                                                                const int* __restrict__ maskOff,
-                                                                const int* __restrict__ blockOff,
-                                                                int* __restrict__ list) {
-  const int64_t m = (int64_t)blockIdx.x * kScanBlock + threadIdx.x;
-  if (m >= nMasks) return;
-  unsigned long long bits = masks[m];
-  int at = blockOff[m / kScanBlock] + maskOff[m];
-  while (bits) {
-    const int bit = __ffsll((long long)bits) - 1;
-    list[at++] = (int)(m * 64 + bit);
-    bits &= bits - 1ull;
-  }
-}
-
-// Compacting solve, phase 2: a persistent grid drains the list.  Each
-// wavefront takes `grab` chunks of 64 list entries at a time (one vector
-// atomic on the grab counter, by lane 0) and continues those zones for the
-// remaining maxNonLinearIter - budget1 updates; it exits once the counter
-// has passed the list length, which every wavefront reaches because the
-// counter only grows and the length is fixed.
+// Compacting solve, phase 2.  Wavefront w of W takes the hand-over masks w,
+// w + W, w + 2W, ... (stragglers cluster in space, so neighbouring masks go
+// to different wavefronts), gathers their zones in a small list in LDS and
+// solves them 64 at a time; what is left at the end runs on fewer lanes.  It
+// needs no list in memory, no prefix sums between the phases (three launches
+// of 5 us) and no shared counter, and every wavefront ends after nMasks / W
+// masks.
 template <class L, int MODE>
 __global__ __launch_bounds__(kDefaultBlock) void newtonPhase2(DevParams prm, grim_zone_batch b,
-                                                              grim_newton_stats st, int budget2,
-                                                              const int* __restrict__ list,
-                                                              int* __restrict__ ctrl, int grab) {
+                                                              grim_newton_stats st, int64_t nMasks,
+                                                              const unsigned long long* __restrict__ masks,
+                                                              const int* __restrict__ updates) {
+  __shared__ int zones[kDefaultBlock / 64][128], left[kDefaultBlock / 64][128];
   const int lane = threadIdx.x & 63;
-  const int total = ctrl[0];
-  for (;;) {
-    int base = 0;
-    if (lane == 0) base = atomicAdd(&ctrl[1], 64 * grab);
-    base = __shfl(base, 0, 64);
-    if (base >= total) break;
-    for (int j = 0; j < grab; j++) {
-      const int idx = base + j * 64 + lane;
-      if (idx < total) solveZone<L, MODE>(prm, b, st, (int64_t)list[idx], budget2, true, true);
+  int* zone = zones[threadIdx.x >> 6];
+  int* rest = left[threadIdx.x >> 6];
+  const int64_t waves = (int64_t)gridDim.x * (blockDim.x >> 6);
+  const int64_t wave = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  auto ordered = [] { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); };
+  auto run = [&](int count) {
+    ordered();
+    int done;
+    if (lane < count)
+      solveZone<L, MODE>(prm, b, st, (int64_t)zone[lane], prm.maxIter, rest[lane], 0, true, done);
+    ordered();
+  };
+  int held = 0;  // zones in the list, below 64 between masks
+  for (int64_t base = 0; base < nMasks; base += waves * 64) {
+    // 64 of the wavefront's masks, one per lane
+    const int64_t m = base + lane * waves + wave;
+    unsigned long long mine = m < nMasks ? masks[m] : 0ull;
+    int mineRest = mine ? prm.maxIter - updates[m] : 0;
+    for (unsigned long long todo = __ballot(mine != 0ull); todo; todo &= todo - 1ull) {
+      const int src = __ffsll((long long)todo) - 1;
+      const unsigned long long mask = __shfl(mine, src, 64);
+      const int r = __shfl(mineRest, src, 64);
+      if ((mask >> lane) & 1ull) {
+        const int at = held + __popcll(mask & ((1ull << lane) - 1ull));
+        zone[at] = (int)((base + src * waves + wave) * 64 + lane);
+        rest[at] = r;
+      }
+      held += __popcll(mask);
+      if (held >= 64) {
+        run(64);
+        held -= 64;
+        if (lane < held) {
+          zone[lane] = zone[64 + lane];
+          rest[lane] = rest[64 + lane];
+        }
+        ordered();
+      }
     }
   }
+  run(held);
 }
 
 template <class L, int MODE>
@@ -628,37 +612,24 @@ __device__ __forceinline__ void fdJacobianFast(const double* P, const double* R,
   }
 }
 
-// Carve-up of the caller's (or the library's) compaction workspace.
+// Carve-up of the caller's (or the library's) compaction workspace: per
+// phase-1 wavefront the zones it hands over and the updates they have had.
 struct CompactionWorkspace {
-  unsigned long long* masks;  // one per phase-1 wavefront
-  int* maskOff;               // popcount prefix within each scan workgroup
-  int* blockSum;              // scan workgroup totals, then their prefix
-  int* list;                  // unconverged zones, ascending
-  int* ctrl;                  // [0] list length, [1] grab counter
+  unsigned long long* masks;
+  int* updates;
 };
 
 constexpr int64_t align256(int64_t x) { return (x + 255) / 256 * 256; }
 
 // Bytes of the workspace for n zones, and the carve-up of a buffer of that size.
 constexpr int64_t compactionBytes(int64_t n) {
-  const int64_t nMasks = (n + 63) / 64, nScan = (nMasks + kScanBlock - 1) / kScanBlock;
-  return align256(nMasks * 8) + align256(nMasks * 4) + align256(nScan * 4) + align256(n * 4) + 256;
+  const int64_t nMasks = (n + 63) / 64;
+  return align256(nMasks * 8) + align256(nMasks * 4) + 256;
 }
 
 inline CompactionWorkspace carveCompaction(void* base, int64_t n) {
-  const int64_t nMasks = (n + 63) / 64, nScan = (nMasks + kScanBlock - 1) / kScanBlock;
-  char* p = (char*)base;
-  CompactionWorkspace w;
-  w.masks = (unsigned long long*)p;
-  p += align256(nMasks * 8);
-  w.maskOff = (int*)p;
-  p += align256(nMasks * 4);
-  w.blockSum = (int*)p;
-  p += align256(nScan * 4);
-  w.list = (int*)p;
-  p += align256(n * 4);
-  w.ctrl = (int*)p;
-  return w;
+  const int64_t nMasks = (n + 63) / 64;
+  return {(unsigned long long*)base, (int*)((char*)base + align256(nMasks * 8))};
 }
 
 // Launch configuration of the per-zone solve (chosen by the autotuner or the
@@ -668,9 +639,8 @@ struct LaunchCfg {
   bool compaction;           // two-phase compacting solve
   bool workgroupSplit;       // one pass, stragglers gathered inside each workgroup (newtonPerZoneSplit)
   int budget1;               // phase-1 update budget
-  int group;                 // phase-2 grab: chunks of 64 list entries per atomic (1..kMaxGroup)
   int persistentWaves;       // phase-2 grid, in wavefronts
-  CompactionWorkspace ws;    // masks, prefix sums, work list, counters
+  CompactionWorkspace ws;    // what phase 1 hands over
 };
 
 // Dynamic LDS of a per-zone solve workgroup of `block` lanes.
@@ -701,25 +671,19 @@ void launchSolve(const DevParams& prm, const grim_zone_batch& b, const grim_newt
     return;
   }
   const CompactionWorkspace& w = cfg.ws;
+  const size_t lds = ldsBytes<L, MODE>(cfg.block);
   if constexpr (MODE == MODE_MIXED) {
     if (fold)
-      newtonPhase1Fold<L, MODE, 3><<<grid, cfg.block, ldsBytes<L, MODE>(cfg.block), s>>>(prm, b, st, cfg.budget1,
-                                                                                        w.masks, *fold);
+      newtonPhase1Fold<L, MODE, 3><<<grid, cfg.block, lds, s>>>(prm, b, st, cfg.budget1, w.masks, w.updates, *fold);
     else
-      newtonPhase1<L, MODE><<<grid, cfg.block, ldsBytes<L, MODE>(cfg.block), s>>>(prm, b, st, cfg.budget1,
-                                                                                 w.masks);
+      newtonPhase1<L, MODE><<<grid, cfg.block, lds, s>>>(prm, b, st, cfg.budget1, w.masks, w.updates);
   } else {
-    newtonPhase1<L, MODE><<<grid, cfg.block, ldsBytes<L, MODE>(cfg.block), s>>>(prm, b, st, cfg.budget1, w.masks);
+    newtonPhase1<L, MODE><<<grid, cfg.block, lds, s>>>(prm, b, st, cfg.budget1, w.masks, w.updates);
   }
   const int64_t nMasks = (b.n + 63) / 64;
-  const int64_t nScan = (nMasks + kScanBlock - 1) / kScanBlock;
-  scanMasksKernel<<<(unsigned)nScan, kScanBlock, 0, s>>>(nMasks, w.masks, w.maskOff, w.blockSum);
-  scanBlocksKernel<<<1, kScanBlock, 0, s>>>(nScan, w.blockSum, w.ctrl);
-  scatterListKernel<<<(unsigned)nScan, kScanBlock, 0, s>>>(nMasks, w.masks, w.maskOff, w.blockSum, w.list);
   const int64_t waves = std::min<int64_t>(cfg.persistentWaves, nMasks);
   const unsigned grid2 = (unsigned)((waves * 64 + cfg.block - 1) / cfg.block);
-  newtonPhase2<L, MODE><<<grid2, cfg.block, ldsBytes<L, MODE>(cfg.block), s>>>(
-      prm, b, st, prm.maxIter - cfg.budget1, w.list, w.ctrl, cfg.group);
+  newtonPhase2<L, MODE><<<grid2, cfg.block, lds, s>>>(prm, b, st, nMasks, w.masks, w.updates);
 }
 
 // Host launcher of the fast translation unit (newton_fast.hip).

@@ -133,9 +133,9 @@ typedef struct grim_newton_opts {
   int jacobian;      /* grim_jacobian_kind */
   int lu_precision;  /* grim_lu_precision */
   int semantics;     /* grim_semantics */
-  int compaction;    /* 1: every zone gets phase1_iters updates, then the
-                        still unconverged zones are compacted into a dense
-                        work list that a persistent kernel drains (at most
+  int compaction;    /* 1: every zone gets phase1_iters updates, wavefronts
+                        with more than a few unconverged zones go on, and a
+                        second kernel gathers the zones left over (at most
                         2^30 zones); 2: one pass in which, after
                         phase1_iters updates, each workgroup gathers its
                         unconverged zones onto its first lanes (no work
@@ -146,10 +146,10 @@ typedef struct grim_newton_opts {
                         multiply-add (bit-reproducible against a CPU FP64
                         evaluation); 1 = fused multiply-adds and reciprocal
                         forms.  The mixed path is always fused. */
-  int phase1_iters;  /* compaction: Newton updates before the work list is
-                        compacted (0 = library default) */
-  int phase2_group;  /* compaction: chunks of 64 work-list zones a phase-2
-                        wavefront takes per grab, 1..8 (0 = default) */
+  int phase1_iters;  /* compaction: Newton updates before a zone may be
+                        handed to the second phase (0 = library default) */
+  int phase2_group;  /* 0..8; has no effect (each phase-2 wavefront takes a
+                        fixed share of the zones left over) */
   void* workspace;   /* compaction: device scratch of at least
                         grim_newton_workspace_bytes(n) bytes, or NULL to let
                         the library allocate it on the stream */
@@ -222,8 +222,8 @@ int grim_batched_newton(const grim_params* p, const grim_zone_batch* b,
  * cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc): it calls no hipMalloc, hipFree or
  * allocating library routine.  The compacting solve (compaction = 1, or
- * GRIM_LU_FP32_FP64) keeps its work list in a library-owned device array of
- * compaction workspace for GRIM_NOALLOC_MAX_ZONES zones (about 35 MB, one
+ * GRIM_LU_FP32_FP64) keeps its hand-over masks in a library-owned device array
+ * of compaction workspace for GRIM_NOALLOC_MAX_ZONES zones (about 1.6 MB, one
  * copy per device, held until the process ends).  Same options and results
  * as grim_batched_newton, except: per-zone semantics only, opts->workspace
  * must be NULL, and at most GRIM_NOALLOC_MAX_ZONES zones (GRIM_ERR_BAD_ARG

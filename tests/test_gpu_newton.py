@@ -370,6 +370,32 @@ def test_compaction_is_bit_identical_to_one_pass(capi, torch_cuda, case):
         np.testing.assert_array_equal(out[0][2], out[c][2])
 
 
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 1000, 20001, 300007])
+@pytest.mark.parametrize("path", ["fd", "mixed", "analytic64"])
+def test_hand_over_between_phases_changes_nothing(capi, torch_cuda, path, n):
+    """The compacting solve at the edges of its hand-over: one zone, a part of
+    a wavefront, one zone beyond it, fewer wavefronts than phase 2 launches
+    and more.  Zones that wavefronts drop at different update counts end as
+    in the one-pass solve, bit for bit, with the same iteration counts."""
+    torch = torch_cuda
+    p, b, rhs, mask = make_problem(capi, torch, n, True, seed=SEED + 5)
+    p.maxNonLinearIter = 9
+    jac = capi.JAC_FD if path == "fd" else capi.JAC_ANALYTIC
+    lu = capi.LU_FP32 if path == "mixed" else capi.LU_FP64
+    out = []
+    for compaction in (0, 1):
+        prim = b["guess"].clone()
+        it = torch.zeros(n, dtype=torch.int32, device="cuda")
+        l2 = torch.zeros(n, dtype=torch.float64, device="cuda")
+        o = capi.newton_opts(jac, lu, compaction=compaction, phase1_iters=1)
+        capi.batched_newton(p, capi.make_batch(prim, b["geom"], rhs, b["prim_old"], None, b["closure"],
+                                               residual_mask=mask), iterations=it, final_l2=l2, opts=o)
+        torch.cuda.synchronize()
+        out.append((host(prim), host(it), host(l2)))
+    for x, y in zip(*out):
+        np.testing.assert_array_equal(x, y)
+
+
 @pytest.mark.parametrize("case", [("fd", False, 0), ("mixed", True, 0), ("mixed", True, 1), ("escalate", True, 1),
                                   ("fd_global", False, 0), ("mixed_noalloc", True, 1)])
 def test_guess_input_equals_copy_then_solve(capi, torch_cuda, case):
