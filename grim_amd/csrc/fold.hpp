@@ -24,6 +24,16 @@ __device__ __forceinline__ void zoneIndex(const Dims& D, int64_t z, int& i, int&
   k = (int)(r / n1);
 }
 
+// timeStepper::computeEMF (constrainedtransport.cpp:49-83) on the X3 edge at
+// the lower corner of zone z, the only edge a two-dimensional grid has.
+template <class L>
+__device__ __forceinline__ double edgeEmf3(const Dims& D, const double* __restrict__ F, int64_t z) {
+#pragma clang fp contract(off)
+  const double* F1B2 = F + (int64_t)L::B2 * D.n;
+  const double* F2B1 = F + (int64_t)(L::DOF + L::B1) * D.n;
+  return 0.25 * (F1B2[z] + F1B2[z - D.s[1]] - F2B1[z] - F2B1[z - D.s[0]]);
+}
+
 // Flux of variable v through the lower face of zone z along d, after
 // timeStepper::fluxCT (constrainedtransport.cpp:3-47) for dim >= 2.
 template <class L, int DIM = 0>
@@ -38,6 +48,12 @@ __device__ __forceinline__ double ctFlux(const Dims& D, const double* __restrict
     const double* e3 = emf + 2 * n;
     const int64_t s1 = D.s[0], s2 = D.s[1], s3 = D.s[2];
     const int b = v - L::B1;
+    if constexpr (DIM == 2) {
+      // each EMF from its four fluxes where it is used: they come from the
+      // caches, and no kernel writes the EMFs first
+      if (d == 0 && b == 1) return 0.5 * (edgeEmf3<L>(D, F, z) + edgeEmf3<L>(D, F, z + s2));
+      if (d == 1 && b == 0) return -0.5 * (edgeEmf3<L>(D, F, z) + edgeEmf3<L>(D, F, z + s1));
+    }
     if (d == 0) {
       if (b == 0) return 0.;
       if (b == 1) return 0.5 * (e3[z] + e3[z + s2]);
@@ -123,8 +139,8 @@ __device__ __forceinline__ void foldZone(const Dims& D, const double* dX, const 
   }
 }
 
-// What a compacting stage solve needs to fold each zone's right-hand side
-// itself (the fold kernel's inputs and outputs).
+// What a stage solve needs to fold each zone's right-hand side itself (the
+// fold kernel's inputs and outputs).
 struct FoldArgs {
   Dims D;
   Box bulk;
@@ -137,20 +153,21 @@ struct FoldArgs {
   const double* consOld;
   const double* sExp;
   const double* sImp;
-  double* rhs;   // written for the zones left to the second phase
+  double* rhs;   // written for every bulk zone, or (compacting solve) for
+                 // the zones left to the second phase
   double* mask;  // the residual mask plane
   // the stage state's field rows (3 planes): zones outside the bulk take
   // them into prim's field rows, so no copy of the rows precedes the solve
   const double* fieldIn;
 };
 
-// Host: whether a grid stage's solve with these options compacts with the
-// mixed analytic Jacobian on a 3D grid, so that its phase 1 can fold the
-// stage's right-hand side itself.
-bool foldFusable(const grim_params& p, const grim_newton_opts& o, int dim);
+// Host: whether a grid stage's solve with these options can fold the stage's
+// right-hand side itself: grim's FD solve and the fused analytic one, per
+// zone, in one pass or (fused) compacting.
+bool foldFusable(const grim_params& p, const grim_newton_opts& o, int64_t n);  // n: zones of the grid
 
-// grim_batched_newton, with the stage fold inside phase 1 when fold is given
-// (then foldFusable must hold).
+// grim_batched_newton, with the stage fold inside the solve when fold is
+// given (then foldFusable must hold).
 int batchedNewton(const grim_params* p, const grim_zone_batch* b, const grim_newton_opts* opts,
                   grim_newton_stats* stats, hipStream_t stream, const FoldArgs* fold);
 

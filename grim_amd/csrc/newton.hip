@@ -342,12 +342,16 @@ using namespace grim;
 
 namespace grim {
 
-bool foldFusable(const grim_params& p, const grim_newton_opts& o, int dim) {
+bool foldFusable(const grim_params& p, const grim_newton_opts& o, int64_t n) {
+  if (o.semantics != GRIM_NEWTON_PER_ZONE) return false;
+  const bool fd = o.jacobian == GRIM_JAC_FD && o.lu_precision == GRIM_LU_FP64 && !o.fused;
   const bool escalate = o.jacobian == GRIM_JAC_ANALYTIC && o.lu_precision == GRIM_LU_FP32_FP64;
   const bool mixed = o.jacobian == GRIM_JAC_ANALYTIC && o.lu_precision == GRIM_LU_FP32;
-  const int budget1 = o.phase1_iters ? o.phase1_iters : 2;
-  return dim == 3 && o.semantics == GRIM_NEWTON_PER_ZONE && (escalate || (mixed && o.compaction == 1)) &&
-         budget1 < p.maxNonLinearIter;
+  // grim's EMHD solve with one lane per zone already spills registers: with
+  // the fold in front it took 200 us on a 65 x 50 x 33 torus against 157 of
+  // the solve, 12 of the fold kernel and 5 of the field copy
+  const bool emhd = p.conduction || p.viscosity;
+  return escalate || (mixed && o.compaction != 2) || (fd && o.compaction == 0 && (!emhd || n <= kWideMaxZones));
 }
 
 int batchedNewton(const grim_params* p, const grim_zone_batch* b, const grim_newton_opts* opts,
@@ -381,7 +385,7 @@ int batchedNewton(const grim_params* p, const grim_zone_batch* b, const grim_new
   if (b->n == 0) return GRIM_OK;
   if (int rc = checkDevice()) return rc;
   hipStream_t s = stream;
-  GRIM_REQUIRE(!fold || foldFusable(*p, o, fold->D.dim), "stage solve: the fold runs inside compacting mixed solves only");
+  GRIM_REQUIRE(!fold || foldFusable(*p, o, b->n), "stage solve: the fold runs inside FD and fused analytic solves only");
   if (o.semantics == GRIM_NEWTON_GLOBAL) {
     // grim's lock-step loop works in prim from the start: copy the guess in
     if (b->guess && b->guess != b->prim)
@@ -420,7 +424,7 @@ int batchedNewton(const grim_params* p, const grim_zone_batch* b, const grim_new
   } else {
     rc = dispatchLayout(*p, [&]<class L>() -> int {
       if (mode == MODE_FD)
-        launchSolve<L, MODE_FD>(prm, bb, st, cfg, s);
+        launchSolve<L, MODE_FD>(prm, bb, st, cfg, s, fold);
       else
         launchSolve<L, MODE_ANALYTIC64>(prm, bb, st, cfg, s);
       return checkLaunch("grim_batched_newton");

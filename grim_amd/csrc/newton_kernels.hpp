@@ -484,13 +484,44 @@ __global__ __launch_bounds__(kDefaultBlock) __attribute__((amdgpu_waves_per_eu(2
   storeHandOver(more, done, z, b.n, masks, updates);
 }
 
-// Phase 1 of a grid stage's compacting solve with the stage fold in front of
-// each zone's Newton iterations: a bulk zone forms its right-hand side, its
-// new field rows and its residual scale from the face fluxes, EMFs, consOld
-// and sources (foldZone, the fold kernel's arithmetic bit for bit), writes
-// the field rows and the mask plane, and keeps the right-hand side in
-// registers; only the zones left unconverged store it for phase 2.  The
-// fold's memory traffic overlaps the solves' arithmetic.
+// The stage fold in front of a zone's Newton iterations: a bulk zone forms
+// its right-hand side, its new field rows and its residual scale from the
+// face fluxes, EMFs, consOld and sources (foldZone, the fold kernel's
+// arithmetic bit for bit), writes the field rows and the mask plane, and
+// keeps the right-hand side in registers.  The fold's memory traffic overlaps
+// the solves' arithmetic, and no fold kernel and no copy of the field rows
+// precede the solve.  `lead`: this lane writes for its zone.
+template <class L, int DIM>
+__device__ __forceinline__ bool foldForSolve(const grim_zone_batch& b, const FoldArgs& f, int64_t z, bool lead,
+                                             double (&rhs)[L::NF], double (&B)[3], double& mask) {
+  const int64_t n = b.n;
+  int i, j, k;
+  zoneIndex(f.D, z, i, j, k);
+  const bool bulk = i >= f.bulk.lo[0] && i < f.bulk.hi[0] && j >= f.bulk.lo[1] && j < f.bulk.hi[1] &&
+                    k >= f.bulk.lo[2] && k < f.bulk.hi[2];
+  mask = 0.;
+#pragma unroll
+  for (int v = 0; v < L::NF; v++) rhs[v] = 0.;
+  B[0] = B[1] = B[2] = 0.;
+  if (bulk) {
+    double rmax;
+    foldZone<L, DIM>(f.D, f.dX, f.F, f.emf, f.geomC, f.consOld, f.sExp, f.sImp, batchDt(b), z, i, j,
+                     f.fluxFilter, rhs, B, rmax);
+    mask = f.scaling ? 1. / rmax : f.mask[z];
+    if (lead) {
+#pragma unroll
+      for (int c = 0; c < 3; c++) b.prim[(L::NF + c) * n + z] = B[c];
+      if (f.scaling) f.mask[z] = mask;
+    }
+  } else if (lead) {
+#pragma unroll
+    for (int c = 0; c < 3; c++) b.prim[(L::NF + c) * n + z] = f.fieldIn[c * n + z];
+  }
+  return bulk;
+}
+
+// Phase 1 of a grid stage's compacting solve with the stage fold; only the
+// zones left unconverged store their right-hand side, for phase 2.
 template <class L, int MODE, int DIM>
 __global__ __launch_bounds__(kDefaultBlock) __attribute__((amdgpu_waves_per_eu(2))) void newtonPhase1Fold(
     DevParams prm, grim_zone_batch b, grim_newton_stats st, int budget1, unsigned long long* __restrict__ masks,
@@ -499,38 +530,32 @@ __global__ __launch_bounds__(kDefaultBlock) __attribute__((amdgpu_waves_per_eu(2
   bool more = false;
   int done = 0;
   if (z < b.n) {
-    const int64_t n = b.n;
-    int i, j, k;
-    zoneIndex(f.D, z, i, j, k);
-    const bool bulk = i >= f.bulk.lo[0] && i < f.bulk.hi[0] && j >= f.bulk.lo[1] && j < f.bulk.hi[1] &&
-                      k >= f.bulk.lo[2] && k < f.bulk.hi[2];
-    double rhs[L::NF], B[3], mask = 0.;
-#pragma unroll
-    for (int v = 0; v < L::NF; v++) rhs[v] = 0.;
-    B[0] = B[1] = B[2] = 0.;
-    if (bulk) {
-      double rmax;
-      foldZone<L, DIM>(f.D, f.dX, f.F, f.emf, f.geomC, f.consOld, f.sExp, f.sImp, batchDt(b), z, i, j,
-                       f.fluxFilter, rhs, B, rmax);
-#pragma unroll
-      for (int c = 0; c < 3; c++) b.prim[(L::NF + c) * n + z] = B[c];
-      if (f.scaling) {
-        mask = 1. / rmax;
-        f.mask[z] = mask;
-      } else {
-        mask = f.mask[z];
-      }
-    } else {
-#pragma unroll
-      for (int c = 0; c < 3; c++) b.prim[(L::NF + c) * n + z] = f.fieldIn[c * n + z];
-    }
+    double rhs[L::NF], B[3], mask;
+    foldForSolve<L, DIM>(b, f, z, true, rhs, B, mask);
     more = solveZone<L, MODE, false, true>(prm, b, st, z, budget1, prm.maxIter, kKeepLanes<MODE>, false, done, rhs, B,
                                            mask);
     if (more)
 #pragma unroll
-      for (int v = 0; v < L::NF; v++) f.rhs[v * n + z] = rhs[v];
+      for (int v = 0; v < L::NF; v++) f.rhs[v * b.n + z] = rhs[v];
   }
   storeHandOver(more, done, z, b.n, masks, updates);
+}
+
+// A grid stage's one-pass solve with the stage fold (WIDE: kWide lanes per
+// zone); the right-hand side of every bulk zone is stored, as the fold kernel
+// leaves it.
+template <class L, int MODE, int DIM, bool WIDE>
+__global__ __launch_bounds__(kDefaultBlock) __attribute__((amdgpu_waves_per_eu(WIDE ? 1 : 2))) void newtonPerZoneFold(
+    DevParams prm, grim_zone_batch b, grim_newton_stats st, FoldArgs f) {
+  const int64_t z = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / (WIDE ? kWide : 1);
+  if (z >= b.n) return;
+  const bool lead = !WIDE || (threadIdx.x % kWide) == 0;
+  double rhs[L::NF], B[3], mask;
+  if (foldForSolve<L, DIM>(b, f, z, lead, rhs, B, mask) && lead)
+#pragma unroll
+    for (int v = 0; v < L::NF; v++) f.rhs[v * b.n + z] = rhs[v];
+  int done;
+  solveZone<L, MODE, WIDE, true>(prm, b, st, z, prm.maxIter, prm.maxIter, 0, false, done, rhs, B, mask);
 }
 
 // Compacting solve, phase 2.  Wavefront w of W takes the hand-over masks w,
@@ -650,13 +675,36 @@ constexpr size_t ldsBytes(int block) {
 }
 
 // Enqueue the per-zone solve of mode MODE on stream s.
-// fold: a grid stage's fold runs inside phase 1 (newtonPhase1Fold; the
-// caller has checked that the solve compacts, see foldFusable).
+// fold: a grid stage's fold runs inside the solve (the caller has checked
+// foldFusable).
 template <class L, int MODE>
 void launchSolve(const DevParams& prm, const grim_zone_batch& b, const grim_newton_stats& st,
                  const LaunchCfg& cfg, hipStream_t s, const FoldArgs* fold = nullptr) {
   const unsigned grid = (unsigned)((b.n + cfg.block - 1) / cfg.block);
+  constexpr bool canFold = MODE == MODE_FD || MODE == MODE_MIXED;
+  // f.operator()<DIM>() for the grid's dimension
+  auto byDim = [&](auto&& f) {
+    if (fold->D.dim == 1) f.template operator()<1>();
+    else if (fold->D.dim == 2) f.template operator()<2>();
+    else f.template operator()<3>();
+  };
   if (!cfg.compaction || cfg.budget1 >= prm.maxIter) {
+    if constexpr (canFold) {
+      if (fold) {
+        byDim([&]<int DIM>() {
+          if constexpr (MODE == MODE_FD) {
+            if (b.n <= kWideMaxZones) {
+              const unsigned wideGrid = (unsigned)((b.n * kWide + kDefaultBlock - 1) / kDefaultBlock);
+              newtonPerZoneFold<L, MODE, DIM, true><<<wideGrid, kDefaultBlock, 0, s>>>(prm, b, st, *fold);
+              return;
+            }
+          }
+          newtonPerZoneFold<L, MODE, DIM, false><<<grid, cfg.block, ldsBytes<L, MODE>(cfg.block), s>>>(prm, b, st,
+                                                                                                      *fold);
+        });
+        return;
+      }
+    }
     if constexpr (MODE == MODE_FD) {
       if (b.n <= kWideMaxZones) {
         const unsigned wideGrid = (unsigned)((b.n * kWide + kDefaultBlock - 1) / kDefaultBlock);
@@ -674,7 +722,9 @@ void launchSolve(const DevParams& prm, const grim_zone_batch& b, const grim_newt
   const size_t lds = ldsBytes<L, MODE>(cfg.block);
   if constexpr (MODE == MODE_MIXED) {
     if (fold)
-      newtonPhase1Fold<L, MODE, 3><<<grid, cfg.block, lds, s>>>(prm, b, st, cfg.budget1, w.masks, w.updates, *fold);
+      byDim([&]<int DIM>() {
+        newtonPhase1Fold<L, MODE, DIM><<<grid, cfg.block, lds, s>>>(prm, b, st, cfg.budget1, w.masks, w.updates, *fold);
+      });
     else
       newtonPhase1<L, MODE><<<grid, cfg.block, lds, s>>>(prm, b, st, cfg.budget1, w.masks, w.updates);
   } else {

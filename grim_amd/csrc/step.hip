@@ -217,6 +217,84 @@ __global__ __launch_bounds__(kBlock) void boundaryKernel(Dims D, Box box, int d,
     if (v < nvars) prim[v * D.n + z] = val[v];
 }
 
+// The ghost zones as six disjoint slabs (X1 sides over the whole grid, X2
+// sides over the bulk X1 range, X3 sides over the bulk X1 and X2 ranges), so
+// that a launch over ghost zones has one thread per zone.
+struct GhostSlabs {
+  Box box[6];
+  int64_t end[6];  // running zone count
+};
+
+inline GhostSlabs ghostSlabs(const Dims& D) {
+  GhostSlabs s;
+  int64_t total = 0;
+  for (int q = 0; q < 6; q++) {
+    const int d = q / 2, side = q % 2;
+    Box& b = s.box[q];
+    for (int e = 0; e < 3; e++) {
+      b.lo[e] = e < d ? D.g[e] : 0;
+      b.hi[e] = e < d ? D.g[e] + D.N[e] : D.NT[e];
+    }
+    b.lo[d] = side == 0 ? 0 : D.g[d] + D.N[d];
+    b.hi[d] = side == 0 ? D.g[d] : D.NT[d];
+    total += b.count();
+    s.end[q] = total;
+  }
+  return s;
+}
+
+// applyBoundaryConditions in one launch, after grid::communicate when `wrap`.
+// The reference fills the sides in turn (communicate, then X1, X2, X3), each
+// from the grid the last one left, so a ghost zone ends as the zone whose
+// out-of-range coordinates are mapped one by one: the first interior layer or
+// the reflected layer along an outflow or mirror direction, the periodic
+// image along a periodic one (`wrap`; left as it is otherwise).  Every such
+// source lies in the bulk along the directions this kernel fills (the caller
+// has N >= numGhost along each), so zones are independent.  One launch where
+// a torus stage had four and a shock tube's two (5 us each on small grids).
+__global__ __launch_bounds__(kBlock) void fillGhostsKernel(Dims D, BcTypes bc, GhostSlabs slabs, int wrap, int nvars,
+                                                           double* __restrict__ prim) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= slabs.end[5]) return;
+  int I[3] = {0, 0, 0};
+  int64_t before = 0;
+#pragma unroll
+  for (int q = 0; q < 6; q++) {
+    if (t >= before && t < slabs.end[q]) slabs.box[q].at(t - before, I[0], I[1], I[2]);
+    before = slabs.end[q];
+  }
+  const int64_t z = flatIndex(D, I[0], I[1], I[2]);
+  bool moved = false;
+#pragma unroll
+  for (int d = 0; d < 3; d++) {
+    const int g = D.g[d], N = D.N[d], a = I[d];
+    const bool lo = a < g, hi = a >= g + N;
+    if (!lo && !hi) continue;
+    const int type = lo ? bc.lo[d] : bc.hi[d];
+    if (type == GRIM_BC_PERIODIC) {
+      if (wrap) {
+        I[d] = lo ? a + N : a - N;
+        moved = true;
+      }
+      continue;
+    }
+    if (type == GRIM_BC_MIRROR)
+      I[d] = lo ? 2 * g - 1 - a : 2 * (N + g) - 1 - a;
+    else
+      I[d] = lo ? g : N + g - 1;
+    moved = true;
+  }
+  if (!moved) return;
+  const int64_t w = flatIndex(D, I[0], I[1], I[2]);
+  double val[GRIM_MAX_VARS];
+#pragma unroll
+  for (int v = 0; v < GRIM_MAX_VARS; v++)
+    if (v < nvars) val[v] = prim[v * D.n + w];
+#pragma unroll
+  for (int v = 0; v < GRIM_MAX_VARS; v++)
+    if (v < nvars) prim[v * D.n + z] = val[v];
+}
+
 // ---------------------------------------------------------------------------
 // Reconstruction and face fluxes
 // ---------------------------------------------------------------------------
@@ -296,13 +374,14 @@ __device__ __forceinline__ void faceState(const StepArgs& a, int64_t z, int64_t 
 // does not cap the occupancy; the left-state wavefronts combine and write
 // every variable of their faces.
 template <class L, int DIR, int RECON>
-__global__ __launch_bounds__(kBlock) void faceFluxSplitKernel(
-    StepArgs a, Box box, const double* __restrict__ prim, const double* __restrict__ geomFace,
-    double* __restrict__ flux, const double* __restrict__ primRight = nullptr) {
-  __shared__ double sh[2 * L::DOF + 2][kFacesPerBlock];
+__device__ __forceinline__ void faceFluxBlock(const StepArgs& a, const Box& box, int64_t block,
+                                              const double* __restrict__ prim,
+                                              const double* __restrict__ geomFace, double* __restrict__ flux,
+                                              const double* __restrict__ primRight,
+                                              double (&sh)[2 * L::DOF + 2][kFacesPerBlock]) {
   const int side = threadIdx.x / kFacesPerBlock;
   const int lf = threadIdx.x % kFacesPerBlock;
-  const int64_t f = (int64_t)blockIdx.x * kFacesPerBlock + lf;
+  const int64_t f = block * kFacesPerBlock + lf;
   const bool active = f < box.count();
   const Dims& D = a.D;
   const int64_t n = D.n;
@@ -344,6 +423,14 @@ __global__ __launch_bounds__(kBlock) void faceFluxSplitKernel(
       flux[v * n + z] = 0.5 * (F[v] + FR - c * (UR - U[v]));
     }
   }
+}
+
+template <class L, int DIR, int RECON>
+__global__ __launch_bounds__(kBlock) void faceFluxSplitKernel(
+    StepArgs a, Box box, const double* __restrict__ prim, const double* __restrict__ geomFace,
+    double* __restrict__ flux, const double* __restrict__ primRight = nullptr) {
+  __shared__ double sh[2 * L::DOF + 2][kFacesPerBlock];
+  faceFluxBlock<L, DIR, RECON>(a, box, blockIdx.x, prim, geomFace, flux, primRight, sh);
 }
 
 // timeStepper::computeEMF (constrainedtransport.cpp:49-83) on the edges the
@@ -471,17 +558,17 @@ __global__ __launch_bounds__(kBlock) void uTKernel(StepArgs a, const double* __r
 // (physics.cpp:360-586) of the stage element; computeImplicitSources of
 // elemOld with the stage element's tau (timestep.cpp:56-60, 211-215); on the
 // half stage also consOld = computeFluxes(0) of elemOld (timestep.cpp:33-36).
-template <class L, int RECON>
-__global__ __launch_bounds__(kBlock) void sourcesKernel(StepArgs a, Box box,
-                                                        const double* __restrict__ prim,
-                                                        const double* __restrict__ primOld,
-                                                        const double* __restrict__ geomC,
-                                                        const double* __restrict__ gamma,
-                                                        const double* __restrict__ uT,
-                                                        double* __restrict__ sExp,
-                                                        double* __restrict__ sImp,
-                                                        double* __restrict__ consOld) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+//
+// INLINE_UT: u_mu and T of the stencil's neighbours are evaluated here from
+// their primitives instead of read from uTKernel's planes (the same
+// kinematics, so the same values): on a small grid the repeated evaluations
+// cost less than the launch they save.
+template <class L, int RECON, bool INLINE_UT>
+__device__ __forceinline__ void sourcesZone(const StepArgs& a, const Box& box, int64_t t,
+                                            const double* __restrict__ prim, const double* __restrict__ primOld,
+                                            const double* __restrict__ geomC, const double* __restrict__ gamma,
+                                            const double* __restrict__ uT, double* __restrict__ sExp,
+                                            double* __restrict__ sImp, double* __restrict__ consOld) {
   if (t >= box.count()) return;
   int i, j, k;
   box.at(t, i, j, k);
@@ -541,22 +628,51 @@ __global__ __launch_bounds__(kBlock) void sourcesKernel(StepArgs a, Box box,
   }
   if constexpr (L::EMHD) {
     auto gam = [&](int l, int p, int q) { return gamma[(l * 16 + p * 4 + q) * ng + zg]; };
-    auto slopeOf = [&](const double* arr, int d) {
-      double y[5];
+    // slopes of u_mu (entries 0..3) and T (entry 4) along each direction:
+    // evaluated up front here, or read plane by plane where they are used
+    double slope[INLINE_UT ? 3 : 1][5];
+    if constexpr (INLINE_UT) {
 #pragma unroll
-      for (int q = 0; q < 5; q++) y[q] = arr[z + (q - 2) * D.s[d]];
-      return slopeZone<RECON>(y, a.theta, a.dX[d]);
+      for (int d = 0; d < 3; d++) {
+#pragma unroll
+        for (int c = 0; c < 5; c++) slope[d][c] = 0.;
+        if (d >= D.dim) continue;
+        double y[5][5];  // [u_0..u_3, T][stencil]
+#pragma unroll
+        for (int q = 0; q < 5; q++) {
+          const int64_t zq = z + (q - 2) * D.s[d];
+          double Pq[L::DOF];
+#pragma unroll
+          for (int v = 0; v < L::DOF; v++) Pq[v] = prim[v * n + zq];
+          ZoneGeom Gq;
+          loadGeom(geomC, ng, geomIndexOf(D, zq), Gq);
+          Kinematics kq;
+          kinematics<L>(Pq, Gq, a.prm, kq);
+#pragma unroll
+          for (int c = 0; c < 4; c++) y[c][q] = kq.uCov[c];
+          y[4][q] = kq.temperature;
+        }
+#pragma unroll
+        for (int c = 0; c < 5; c++) slope[d][c] = slopeZone<RECON>(y[c], a.theta, a.dX[d]);
+      }
+    }
+    auto slopeOf = [&](int c, int d) {
+      if constexpr (INLINE_UT) {
+        return slope[d][c];
+      } else {
+        double y[5];
+#pragma unroll
+        for (int q = 0; q < 5; q++) y[q] = uT[c * n + z + (q - 2) * D.s[d]];
+        return slopeZone<RECON>(y, a.theta, a.dX[d]);
+      }
     };
     double graduCov[4][4];
 #pragma unroll
     for (int mu = 0; mu < 4; mu++) {
-      const double* um = uT + mu * n;
       graduCov[0][mu] = 0.;
-      graduCov[1][mu] = slopeOf(um, 0);
-      graduCov[2][mu] = 0.;
-      if (D.dim > 1) graduCov[2][mu] = slopeOf(um, 1);
-      graduCov[3][mu] = 0.;
-      if (D.dim > 2) graduCov[3][mu] = slopeOf(um, 2);
+      graduCov[1][mu] = slopeOf(mu, 0);
+      graduCov[2][mu] = D.dim > 1 ? slopeOf(mu, 1) : 0.;
+      graduCov[3][mu] = D.dim > 2 ? slopeOf(mu, 2) : 0.;
 #pragma unroll
       for (int nu = 0; nu < 4; nu++)
 #pragma unroll
@@ -582,14 +698,7 @@ __global__ __launch_bounds__(kBlock) void sourcesKernel(StepArgs a, Box box,
       src[L::DP] = sd;
     }
     if constexpr (L::COND_ON) {
-      const double* Tp = uT + 4 * n;
-      double gradT[4];
-      gradT[0] = 0.;
-      gradT[1] = slopeOf(Tp, 0);
-      gradT[2] = 0.;
-      if (D.dim > 1) gradT[2] = slopeOf(Tp, 1);
-      gradT[3] = 0.;
-      if (D.dim > 2) gradT[3] = slopeOf(Tp, 2);
+      const double gradT[4] = {0., slopeOf(4, 0), D.dim > 1 ? slopeOf(4, 1) : 0., D.dim > 2 ? slopeOf(4, 2) : 0.};
       double q0 = 0.;
 #pragma unroll
       for (int mu = 0; mu < 4; mu++) {
@@ -614,6 +723,20 @@ __global__ __launch_bounds__(kBlock) void sourcesKernel(StepArgs a, Box box,
   }
 #pragma unroll
   for (int v = 0; v < L::NF; v++) sExp[v * n + z] = src[v];
+}
+
+template <class L, int RECON>
+__global__ __launch_bounds__(kBlock) void sourcesKernel(StepArgs a, Box box,
+                                                        const double* __restrict__ prim,
+                                                        const double* __restrict__ primOld,
+                                                        const double* __restrict__ geomC,
+                                                        const double* __restrict__ gamma,
+                                                        const double* __restrict__ uT,
+                                                        double* __restrict__ sExp,
+                                                        double* __restrict__ sImp,
+                                                        double* __restrict__ consOld) {
+  sourcesZone<L, RECON, false>(a, box, (int64_t)blockIdx.x * blockDim.x + threadIdx.x, prim, primOld, geomC, gamma, uT,
+                               sExp, sImp, consOld);
 }
 
 // ---------------------------------------------------------------------------
@@ -782,11 +905,9 @@ __global__ __launch_bounds__(kBlock) void dtKernel(StepArgs a, const double* __r
 // clock[0] = time, clock[1] = dt, clock[2] = dt/2 (the half stage's dt').
 enum { CLOCK_TIME = 0, CLOCK_DT = 1, CLOCK_HALF_DT = 2, CLOCK_WORDS = 4 };
 
-__global__ __launch_bounds__(kBlock) void maxReduceKernel(int64_t count, const double* __restrict__ in,
-                                                          double* __restrict__ out,
-                                                          double* __restrict__ clock = nullptr,
-                                                          double courant = 0., double maxIncrement = 0.) {
-  __shared__ double red[kBlock];
+__device__ __forceinline__ void maxReduceBlock(double* red, int64_t count, const double* __restrict__ in,
+                                               double* __restrict__ out, double* __restrict__ clock, double courant,
+                                               double maxIncrement) {
   double m = -INFINITY;
   for (int64_t t = threadIdx.x; t < count; t += kBlock) m = stdmax(m, in[t]);
   red[threadIdx.x] = m;
@@ -805,6 +926,50 @@ __global__ __launch_bounds__(kBlock) void maxReduceKernel(int64_t count, const d
       clock[CLOCK_DT] = newDt;
       clock[CLOCK_HALF_DT] = newDt / 2.;
     }
+  }
+}
+
+__global__ __launch_bounds__(kBlock) void maxReduceKernel(int64_t count, const double* __restrict__ in,
+                                                          double* __restrict__ out,
+                                                          double* __restrict__ clock = nullptr,
+                                                          double courant = 0., double maxIncrement = 0.) {
+  __shared__ double red[kBlock];
+  maxReduceBlock(red, count, in, out, clock, courant, maxIncrement);
+}
+
+// The explicit half of a small grid's stage in one launch: the workgroups of
+// the sources, of the face fluxes of each direction and, on the half stage,
+// one that reduces the step's dt.  They are independent given the stage state
+// (dt is first read by the solve), each runs the code of its own kernel, and
+// on a small grid each kernel alone leaves most of the chip idle and costs a
+// launch (about 5 us back to back).
+struct ExplicitLaunch {
+  Box bulk, face[3];
+  unsigned end[4];  // running workgroup count: sources, X1, X2, X3 faces
+  const double *prim, *primOld, *geomC, *gamma, *geomFace[3];
+  double *sExp, *sImp, *consOld, *flux;
+  // dt: partial maxima and the clock (null on the full stage)
+  const double* dtPart;
+  double *dtOut, *clock;
+  int64_t dtCount;
+  double courant, maxIncrement;
+};
+
+template <class L, int RECON, int DIM>
+__global__ __launch_bounds__(kBlock) void explicitStageKernel(StepArgs a, ExplicitLaunch e) {
+  __shared__ double sh[2 * L::DOF + 2][kFacesPerBlock];
+  const unsigned g = blockIdx.x;
+  const size_t plane = (size_t)L::DOF * a.D.n;
+  if (g < e.end[0]) {
+    sourcesZone<L, RECON, true>(a, e.bulk, (int64_t)g * blockDim.x + threadIdx.x, e.prim, e.primOld, e.geomC, e.gamma,
+                                nullptr, e.sExp, e.sImp, e.consOld);
+  } else if (g < e.end[1]) {
+    faceFluxBlock<L, 0, RECON>(a, e.face[0], g - e.end[0], e.prim, e.geomFace[0], e.flux, nullptr, sh);
+  } else if (DIM > 1 && g < e.end[2]) {
+    if constexpr (DIM > 1)
+      faceFluxBlock<L, 1, RECON>(a, e.face[1], g - e.end[1], e.prim, e.geomFace[1], e.flux + plane, nullptr, sh);
+  } else {
+    maxReduceBlock(&sh[0][0], e.dtCount, e.dtPart, e.dtOut, e.clock, e.courant, e.maxIncrement);
   }
 }
 
@@ -1109,13 +1274,15 @@ __global__ __launch_bounds__(kBlock) void scaleFieldKernel(int64_t n, grim_torus
 }
 
 template <class L>
-__global__ __launch_bounds__(kBlock) void floorKernel(StepArgs a, grim_torus_params t,
+__global__ __launch_bounds__(kBlock) void floorKernel(StepArgs a, Box box, grim_torus_params t,
                                                       const double* __restrict__ geomC,
                                                       const double* __restrict__ floors,
                                                       double* __restrict__ prim) {
-  const int64_t z = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t n = a.D.n;
-  if (z >= n) return;
+  const int64_t tt = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (tt >= box.count()) return;
+  int i, j, k;
+  box.at(tt, i, j, k);
+  const int64_t n = a.D.n, z = flatIndex(a.D, i, j, k);
   double P[L::DOF];
 #pragma unroll
   for (int v = 0; v < L::DOF; v++) P[v] = prim[v * n + z];
@@ -1158,8 +1325,15 @@ __global__ __launch_bounds__(kBlock) void nanZeroKernel(int64_t n, int nvars, co
 // the next computeDt's per-workgroup maxima of the inverse time step of the
 // result (timestep.cpp:336-391), which the next step's reduction reads.
 // Each value is the separate kernels' bit for bit.
-template <class L, bool TORUS>
-__global__ __launch_bounds__(kBlock) void endStepKernel(StepArgs a, grim_torus_params t,
+//
+// COMM: grid::communicate of the result first, in the same pass.  Off the
+// torus the bulk is not written here, so a ghost zone reads its periodic
+// image (or takes the zeros outside the domain) itself.  On the torus the
+// bulk is floored in place; only X3 is periodic there (the caller has checked
+// it), where an image shares its source's geometry and so its floors, and
+// the source's thread writes the images.
+template <class L, bool TORUS, bool COMM>
+__global__ __launch_bounds__(kBlock) void endStepKernel(StepArgs a, grim_torus_params t, BcTypes bc,
                                                         const double* __restrict__ geomC,
                                                         const double* __restrict__ floors,
                                                         const unsigned long long* __restrict__ nanCount,
@@ -1171,10 +1345,42 @@ __global__ __launch_bounds__(kBlock) void endStepKernel(StepArgs a, grim_torus_p
   const int64_t n = a.D.n;
   if (z == 0) clock[CLOCK_TIME] += clock[CLOCK_DT];
   double m = -INFINITY;
-  if (z < n) {
+  bool mine = z < n, outside = false, ghost = false;
+  int64_t src = z, image[2] = {-1, -1};
+  if constexpr (COMM) {
+    if (mine) {
+      int I[3];
+      zoneIndex(a.D, z, I[0], I[1], I[2]);
+      const int k = I[2];
+#pragma unroll
+      for (int d = 0; d < 3; d++) {
+        const int g = a.D.g[d], N = a.D.N[d];
+        if (I[d] < g) {
+          outside = outside || bc.lo[d] != GRIM_BC_PERIODIC;
+          I[d] += N;
+          ghost = true;
+        } else if (I[d] >= g + N) {
+          outside = outside || bc.hi[d] != GRIM_BC_PERIODIC;
+          I[d] -= N;
+          ghost = true;
+        }
+      }
+      if constexpr (TORUS) {
+        if (ghost && !outside) mine = false;
+        if (!ghost && a.D.g[2] > 0) {
+          const int N = a.D.N[2];
+          if (k >= N && bc.lo[2] == GRIM_BC_PERIODIC) image[0] = z - N * a.D.s[2];
+          if (k + N < a.D.NT[2] && bc.hi[2] == GRIM_BC_PERIODIC) image[1] = z + N * a.D.s[2];
+        }
+      } else if (ghost && !outside) {
+        src = flatIndex(a.D, I[0], I[1], I[2]);
+      }
+    }
+  }
+  if (mine) {
     double P[L::DOF];
 #pragma unroll
-    for (int v = 0; v < L::DOF; v++) P[v] = prim[v * n + z];
+    for (int v = 0; v < L::DOF; v++) P[v] = COMM && outside ? 0. : prim[v * n + src];
     GeomFull G;
     loadGeomFull(geomC, a.D.ng, geomIndexOf(a.D, z), G);
     if constexpr (TORUS) {
@@ -1190,9 +1396,20 @@ __global__ __launch_bounds__(kBlock) void endStepKernel(StepArgs a, grim_torus_p
     }
 #pragma unroll
     for (int v = 0; v < L::DOF; v++) {
-      if constexpr (TORUS) prim[v * n + z] = P[v];
+      if (TORUS || (COMM && ghost)) prim[v * n + z] = P[v];
       primOld[v * n + z] = P[v];
       primDt[v * n + z] = P[v];
+    }
+    if constexpr (TORUS && COMM) {
+#pragma unroll
+      for (int q = 0; q < 2; q++)
+        if (image[q] >= 0)
+#pragma unroll
+          for (int v = 0; v < L::DOF; v++) {
+            prim[v * n + image[q]] = P[v];
+            primOld[v * n + image[q]] = P[v];
+            primDt[v * n + image[q]] = P[v];
+          }
     }
     m = zoneInvDt<L>(a, P, G);
   }
@@ -1325,16 +1542,20 @@ __global__ __launch_bounds__(kBlock) void obsFinishKernel(const double* __restri
   if (t < OBS_WORDS) out[t] = sh[t][0];
 }
 
-// inflowCheck (:941-1044) on the radial ghost slabs.
+// inflowCheck (:941-1044) on both radial ghost slabs.
 template <class L>
-__global__ __launch_bounds__(kBlock) void inflowCheckKernel(StepArgs a, grim_torus_params t, Box box, int side,
+__global__ __launch_bounds__(kBlock) void inflowCheckKernel(StepArgs a, grim_torus_params t, Box box,
                                                             const double* __restrict__ geomC,
                                                             double* __restrict__ prim) {
+  // box: the inner slab; the outer one is the same box N1 + numGhost further
   const int64_t tt = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (tt >= box.count()) return;
-  int i, j, k;
-  box.at(tt, i, j, k);
+  const int64_t count = box.count();
+  if (tt >= 2 * count) return;
+  const int side = tt >= count ? 1 : 0;
   const Dims& D = a.D;
+  int i, j, k;
+  box.at(side ? tt - count : tt, i, j, k);
+  if (side) i += D.N[0] + D.g[0];
   const int64_t n = D.n, z = flatIndex(D, i, j, k);
   double P[L::DOF];
 #pragma unroll
@@ -1465,6 +1686,40 @@ int withLayout(const grim_ctx* x, F&& f) {
   return dispatchLayout(x->p, std::forward<F>(f));
 }
 
+Box wholeBox(const Dims& D) {
+  Box b;
+  for (int d = 0; d < 3; d++) {
+    b.lo[d] = 0;
+    b.hi[d] = D.NT[d];
+  }
+  return b;
+}
+
+BcTypes boundaryTypes(const grim_ctx* x) {
+  return {{x->c.boundaryLeft, x->c.boundaryBottom, x->c.boundaryBack},
+          {x->c.boundaryRight, x->c.boundaryTop, x->c.boundaryFront}};
+}
+
+// Every ghost zone's source lies in the bulk: fillGhostsKernel and the
+// communicate of endStepKernel apply.
+bool ghostsFromBulk(const Dims& D) {
+  for (int d = 0; d < D.dim; d++)
+    if (D.N[d] < D.g[d]) return false;
+  return true;
+}
+
+// The step's communicates run inside the kernels that follow them (the next
+// stage's ghost fill, the end of the step); on the torus when only X3 is
+// periodic, where an image has its source's geometry and floors.
+bool communicateFolds(const grim_ctx* x) {
+  if (!ghostsFromBulk(x->D)) return false;
+  if (!x->torus) return true;
+  const BcTypes bc = boundaryTypes(x);
+  for (int d = 0; d < 2; d++)
+    if (bc.lo[d] == GRIM_BC_PERIODIC || bc.hi[d] == GRIM_BC_PERIODIC) return false;
+  return true;
+}
+
 Box bulkBox(const Dims& D) {
   Box b;
   for (int d = 0; d < 3; d++) {
@@ -1498,15 +1753,20 @@ Box edgeBox(const Dims& D) {
 
 int applyBoundaries(grim_ctx* x, double* prim, int nvars, bool periodicFill) {
   const Dims& D = x->D;
-  BcTypes bc;
-  const int lo[3] = {x->c.boundaryLeft, x->c.boundaryBottom, x->c.boundaryBack};
-  const int hi[3] = {x->c.boundaryRight, x->c.boundaryTop, x->c.boundaryFront};
-  for (int d = 0; d < 3; d++) {
-    bc.lo[d] = lo[d];
-    bc.hi[d] = hi[d];
+  const BcTypes bc = boundaryTypes(x);
+  if (ghostsFromBulk(D)) {
+    bool any = periodicFill;
+    for (int d = 0; d < D.dim; d++)
+      any = any || bc.lo[d] != GRIM_BC_PERIODIC || bc.hi[d] != GRIM_BC_PERIODIC;
+    const GhostSlabs slabs = ghostSlabs(D);
+    if (any && slabs.end[5] > 0)
+      fillGhostsKernel<<<blocksFor(slabs.end[5]), kBlock, 0, x->s>>>(D, bc, slabs, periodicFill ? 1 : 0, nvars, prim);
+    return checkLaunch("boundaries");
   }
+  // grids thinner than the ghost layer: side by side, each from what the last
+  // one left
   if (periodicFill) communicateKernel<<<blocksFor(D.n), kBlock, 0, x->s>>>(D, bc, nvars, prim);
-  const int types[6] = {lo[0], hi[0], lo[1], hi[1], lo[2], hi[2]};
+  const int types[6] = {bc.lo[0], bc.hi[0], bc.lo[1], bc.hi[1], bc.lo[2], bc.hi[2]};
   for (int d = 0; d < D.dim; d++)
     for (int side = 0; side < 2; side++) {
       const int type = types[2 * d + side];
@@ -1524,13 +1784,7 @@ int applyBoundaries(grim_ctx* x, double* prim, int nvars, bool periodicFill) {
 }
 
 int communicate(grim_ctx* x, double* prim, int nvars) {
-  BcTypes bc;
-  const int lo[3] = {x->c.boundaryLeft, x->c.boundaryBottom, x->c.boundaryBack};
-  const int hi[3] = {x->c.boundaryRight, x->c.boundaryTop, x->c.boundaryFront};
-  for (int d = 0; d < 3; d++) {
-    bc.lo[d] = lo[d];
-    bc.hi[d] = hi[d];
-  }
+  const BcTypes bc = boundaryTypes(x);
   communicateKernel<<<blocksFor(x->D.n), kBlock, 0, x->s>>>(x->D, bc, nvars, prim);
   return checkLaunch("communicate");
 }
@@ -1587,7 +1841,9 @@ int fluxesAndEmf(grim_ctx* x, const double* prim, bool allFaces) {
   launchFace<L, 0>(x, prim, x->fluxes, allFaces);
   if (x->D.dim > 1) launchFace<L, 1>(x, prim, x->fluxes + plane, allFaces);
   if (x->D.dim > 2) launchFace<L, 2>(x, prim, x->fluxes + 2 * plane, allFaces);
-  if (x->D.dim > 1) {
+  // below three dimensions the divergence forms its EMFs itself; only the
+  // flux arrays handed out after flux-CT read the planes there
+  if (x->D.dim > 2 || (x->D.dim > 1 && allFaces)) {
     const Box e = edgeBox(x->D);
     emfKernel<L><<<blocksFor(e.count()), kBlock, 0, x->s>>>(x->D, e, x->fluxes, x->emf);
   }
@@ -1618,6 +1874,62 @@ int explicitSources(grim_ctx* x, const double* prim, const double* primOld, doub
                                                                  x->uT, sExp, sImp, consOld);
   }
   return checkLaunch("sources");
+}
+
+// Whether a stage's explicit half runs as one launch: below three dimensions
+// (where the EMHD sources evaluate few neighbours), in grim's order, on grids
+// whose kernels are launches rather than work.  kOneLaunchZones: on a 256 x
+// 256 vortex (68,644 zones) sources and faces took 6 + 11 + 11 us as three
+// launches and take 17 us as one, on a 64 x 64 wave 4 + 8 + 8 and 7.5 us; a
+// larger grid fills the chip with each, and the joint kernel's registers (the
+// sources') would lower the faces' occupancy.
+constexpr int64_t kOneLaunchZones = 1 << 17;
+bool explicitInOneLaunch(const grim_ctx* x) {
+  return x->D.dim < 3 && !x->c.explicitFast && x->D.n <= kOneLaunchZones;
+}
+
+// The explicit half of stage st in one launch (explicitStageKernel); reduceDt:
+// with the step's dt from the partial maxima the last step left.
+template <class L>
+int explicitStage(grim_ctx* x, int st, const double* prim, bool reduceDt) {
+  ExplicitLaunch e = {};
+  e.bulk = bulkBox(x->D);
+  e.end[0] = blocksFor(e.bulk.count());
+  const double* gf[3] = {x->geomX1, x->geomX2, x->geomC};
+  for (int d = 0; d < 3; d++) {
+    e.end[d + 1] = e.end[d];
+    if (d >= x->D.dim) continue;
+    e.face[d] = stageFaceBox(x->D, d);
+    e.geomFace[d] = gf[d];
+    e.end[d + 1] += (unsigned)((e.face[d].count() + kFacesPerBlock - 1) / kFacesPerBlock);
+  }
+  e.prim = prim;
+  e.primOld = x->primOld;
+  e.geomC = x->geomC;
+  e.gamma = x->gamma;
+  e.sExp = x->sExp;
+  e.sImp = L::EMHD ? x->sImp : nullptr;
+  e.consOld = st == 0 ? x->consOld : nullptr;
+  e.flux = x->fluxes;
+  if (reduceDt) {
+    e.dtCount = blocksFor(x->D.n);
+    e.dtPart = x->dtPart;
+    e.dtOut = x->dtPart + e.dtCount;
+    e.clock = x->clock;
+    e.courant = x->c.CourantFactor;
+    e.maxIncrement = x->c.maxDtIncrement;
+  }
+  const unsigned nb = e.end[3] + (reduceDt ? 1 : 0);
+  auto go = [&]<int RECON>() {
+    if (x->D.dim == 1)
+      explicitStageKernel<L, RECON, 1><<<nb, kBlock, 0, x->s>>>(x->a, e);
+    else
+      explicitStageKernel<L, RECON, 2><<<nb, kBlock, 0, x->s>>>(x->a, e);
+  };
+  if (x->c.reconstruction == GRIM_RECON_WENO5) go.template operator()<GRIM_RECON_WENO5>();
+  else if (x->c.reconstruction == GRIM_RECON_PPM) go.template operator()<GRIM_RECON_PPM>();
+  else go.template operator()<GRIM_RECON_MINMOD>();
+  return checkLaunch("explicit stage");
 }
 
 // max over zones of the inverse time step, into x->red[nb] (device); with
@@ -1654,7 +1966,8 @@ int computeDtOnDevice(grim_ctx* x, const double* prim) {
 
 template <class L>
 int applyFloor(grim_ctx* x, double* prim) {
-  floorKernel<L><<<blocksFor(x->D.n), kBlock, 0, x->s>>>(x->a, x->tp, x->geomC, x->floors, prim);
+  const Box b = wholeBox(x->D);
+  floorKernel<L><<<blocksFor(b.count()), kBlock, 0, x->s>>>(x->a, b, x->tp, x->geomC, x->floors, prim);
   return checkLaunch("applyFloor");
 }
 
@@ -1811,16 +2124,9 @@ __global__ __launch_bounds__(kBlock) void sideStateKernel(Dims D, const double* 
 template <class L>
 int torusBCs(grim_ctx* x, double* prim) {
   const Dims& D = x->D;
-  for (int side = 0; side < 2; side++) {
-    Box b;
-    for (int d = 0; d < 3; d++) {
-      b.lo[d] = 0;
-      b.hi[d] = D.NT[d];
-    }
-    b.lo[0] = side == 0 ? 0 : D.N[0] + D.g[0];
-    b.hi[0] = side == 0 ? D.g[0] : D.N[0] + 2 * D.g[0];
-    inflowCheckKernel<L><<<blocksFor(b.count()), kBlock, 0, x->s>>>(x->a, x->tp, b, side, x->geomC, prim);
-  }
+  Box b = wholeBox(D);
+  b.hi[0] = D.g[0];
+  inflowCheckKernel<L><<<blocksFor(2 * b.count()), kBlock, 0, x->s>>>(x->a, x->tp, b, x->geomC, prim);
   if (D.dim >= 2) {
     const int64_t cols = 2 * (int64_t)D.NT[0] * D.NT[2];
     fixPolesKernel<L><<<blocksFor(cols), kBlock, 0, x->s>>>(D, x->geomC, prim);
@@ -1851,15 +2157,25 @@ inline const double* stageDtPrime(grim_ctx* x, int st) {
 // stage state (grim_zone_batch.guess), so only the B rows are copied here;
 // the stage-level entry points, whose caller may solve another buffer or
 // inspect the guess, get the whole state copied.
-// foldInSolve: the stage's compacting solve folds each zone's right-hand
-// side itself (newtonPhase1Fold), so no fold kernel runs here.
+// foldInSolve: the stage's solve folds each zone's right-hand side itself
+// (newtonPhase1Fold, newtonPerZoneFold), so no fold kernel runs here.
+// wrap: the stage state still lacks its communicate (the grid step's half
+// stage left it to this ghost fill).  reduceDt: the step's dt comes first.
 template <class L>
-int stagePrepare(grim_ctx* x, int st, bool guessInSolve = false, bool foldInSolve = false) {
+int stagePrepare(grim_ctx* x, int st, bool guessInSolve = false, bool foldInSolve = false, bool wrap = false,
+                 bool reduceDt = false) {
   const Dims& D = x->D;
   const size_t bytes = sizeof(double) * (size_t)L::DOF * D.n;
   double* primStage = stageIn(x, st);
   double* out = stageOut(x, st);
-  if (int rc = applyBoundaries(x, primStage, L::DOF, false)) return rc;
+  const bool oneLaunch = foldInSolve && explicitInOneLaunch(x);
+  if (reduceDt && !oneLaunch) {
+    const unsigned nb = blocksFor(D.n);
+    maxReduceKernel<<<1, kBlock, 0, x->s>>>(nb, x->dtPart, x->dtPart + nb, x->clock, x->c.CourantFactor,
+                                            x->c.maxDtIncrement);
+    if (int rc = checkLaunch("computeDt")) return rc;
+  }
+  if (int rc = applyBoundaries(x, primStage, L::DOF, wrap)) return rc;
   if (x->torus)
     if (int rc = torusBCs<L>(x, primStage)) return rc;
   // grim calls the hook in both stages, but it writes primOld: only the half
@@ -1874,6 +2190,7 @@ int stagePrepare(grim_ctx* x, int st, bool guessInSolve = false, bool foldInSolv
     sideStateKernel<L><<<blocksFor(count), kBlock, 0, x->s>>>(D, x->sideState, primStage);
     if (int rc = checkLaunch("X1 side state")) return rc;
   }
+  if (oneLaunch) return explicitStage<L>(x, st, primStage, reduceDt);
   if (int rc = explicitSources<L>(x, primStage, x->primOld, x->sExp, L::EMHD ? x->sImp : nullptr,
                                   st == 0 ? x->consOld : nullptr))
     return rc;
@@ -1895,10 +2212,10 @@ int stagePrepare(grim_ctx* x, int st, bool guessInSolve = false, bool foldInSolv
   return checkLaunch("fold");
 }
 
-// The stage solve folds in phase 1 when its options compact with the mixed
-// analytic Jacobian on a 3D grid (the grid-step path only: the stage-level
-// entry points keep the separate fold, whose rhs the caller may read).
-bool foldInSolve(const grim_ctx* x) { return foldFusable(x->p, x->opts, x->D.dim); }
+// The stage solve folds the right-hand side itself where its options allow
+// (the grid-step path only: the stage-level entry points keep the separate
+// fold).
+bool foldInSolve(const grim_ctx* x) { return foldFusable(x->p, x->opts, x->D.n); }
 
 // The stage's implicit system as a batch of independent zones (the frozen
 // terms folded into rhs; elemOld = primOld, the coefficient element primOld
@@ -1976,23 +2293,18 @@ int stageFinish(grim_ctx* x, int st) {
   return GRIM_OK;
 }
 
-template <class L>
-int stage(grim_ctx* x, int st, grim_step_stats* stats) {
-  const bool fold = foldInSolve(x);
-  if (int rc = stagePrepare<L>(x, st, true, fold)) return rc;
-  if (int rc = stageSolve(x, st, stageOut(x, st), stageIn(x, st), fold)) return rc;
-  if (stats)
-    if (int rc = stageStats(x, st, stats)) return rc;
-  return stageFinish<L>(x, st);
+template <class L, bool TORUS, bool COMM>
+void launchEndStep(grim_ctx* x) {
+  endStepKernel<L, TORUS, COMM><<<blocksFor(x->D.n), kBlock, 0, x->s>>>(
+      x->a, x->tp, boundaryTypes(x), x->geomC, x->floors, x->counters, x->primNew, x->primOld, x->primDt, x->clock,
+      x->dtPart);
 }
 
 // The end of timeStepper::timeStep: primOld = the full stage's result, the
 // state the next computeDt reads, and time += dt (timestep.cpp:290-300).
 template <class L>
 int stepEnd(grim_ctx* x) {
-  endStepKernel<L, false><<<blocksFor(x->D.n), kBlock, 0, x->s>>>(x->a, x->tp, x->geomC, x->floors, x->counters,
-                                                                  x->primNew, x->primOld, x->primDt, x->clock,
-                                                                  x->dtPart);
+  launchEndStep<L, false, false>(x);
   return checkLaunch("end of step");
 }
 
@@ -2001,17 +2313,32 @@ int stepEnd(grim_ctx* x) {
 // maxima): stageFinish(1) followed by stepEnd.
 template <class L>
 int finishStep(grim_ctx* x) {
-  if (int rc = communicate(x, x->primNew, L::DOF)) return rc;
+  const bool comm = communicateFolds(x);
+  if (!comm)
+    if (int rc = communicate(x, x->primNew, L::DOF)) return rc;
   if (x->torus) {
     const Box b = bulkBox(x->D);
     zeroCountersKernel<<<1, 64, 0, x->s>>>(x->counters, 1);
     nanCountKernel<<<blocksFor(b.count()), kBlock, 0, x->s>>>(x->D, b, L::DOF, x->primNew, x->counters);
-    endStepKernel<L, true><<<blocksFor(x->D.n), kBlock, 0, x->s>>>(x->a, x->tp, x->geomC, x->floors, x->counters,
-                                                                   x->primNew, x->primOld, x->primDt, x->clock,
-                                                                   x->dtPart);
-    return checkLaunch("end of step");
+    if (comm) launchEndStep<L, true, true>(x);
+    else launchEndStep<L, true, false>(x);
+  } else if (comm) {
+    launchEndStep<L, false, true>(x);
+  } else {
+    launchEndStep<L, false, false>(x);
   }
-  return stepEnd<L>(x);
+  return checkLaunch("end of step");
+}
+
+// The half stage's finish: communicate and, on the torus, the floors -- of
+// the bulk alone when the next stage's ghost fill (wrap) does the communicate.
+template <class L>
+int finishHalfStage(grim_ctx* x) {
+  if (!communicateFolds(x)) return stageFinish<L>(x, 0);
+  if (!x->torus) return GRIM_OK;
+  const Box b = bulkBox(x->D);
+  floorKernel<L><<<blocksFor(b.count()), kBlock, 0, x->s>>>(x->a, b, x->tp, x->geomC, x->floors, x->primHalf);
+  return checkLaunch("applyFloor");
 }
 
 int validConfig(const grim_params* p, const grim_grid_config* c) {
@@ -2296,14 +2623,14 @@ int grim_time_step(grim_ctx* x, grim_step_stats* stats) {
   GRIM_REQUIRE(x && x->clockSet, "grim_time_step: no context or dt not set (grim_set_time)");
   return withLayout(x, [&]<class L>() -> int {
     // computeDt of primDt from the partial maxima the previous step's end
-    // (or grim_set_time) left
-    const unsigned nb = blocksFor(x->D.n);
-    maxReduceKernel<<<1, kBlock, 0, x->s>>>(nb, x->dtPart, x->dtPart + nb, x->clock, x->c.CourantFactor,
-                                            x->c.maxDtIncrement);
-    if (int rc = checkLaunch("computeDt")) return rc;
-    if (int rc = stage<L>(x, 0, stats)) return rc;
+    // (or grim_set_time) left, then the half and the full stage
     const bool fold = foldInSolve(x);
-    if (int rc = stagePrepare<L>(x, 1, true, fold)) return rc;
+    if (int rc = stagePrepare<L>(x, 0, true, fold, false, true)) return rc;
+    if (int rc = stageSolve(x, 0, x->primHalf, x->primOld, fold)) return rc;
+    if (stats)
+      if (int rc = stageStats(x, 0, stats)) return rc;
+    if (int rc = finishHalfStage<L>(x)) return rc;
+    if (int rc = stagePrepare<L>(x, 1, true, fold, communicateFolds(x))) return rc;
     if (int rc = stageSolve(x, 1, x->primNew, x->primHalf, fold)) return rc;
     if (stats)
       if (int rc = stageStats(x, 1, stats)) return rc;

@@ -869,6 +869,80 @@ def test_torus_time_step_equals_its_stages(torch, fast):
     staged.close()
 
 
+STEP_CASES = {
+    # dim, (N1, N2, N3), boundaries per direction, reconstruction, EMHD
+    "1d_outflow_emhd": (1, (64, 1, 1), "o", 0, True),
+    "1d_periodic_ideal_weno": (1, (5, 1, 1), "p", 1, False),
+    "2d_periodic_ideal_weno": (2, (17, 33, 1), "pp", 1, False),
+    "2d_mirror_outflow_emhd_ppm": (2, (20, 9, 1), "mo", 2, True),
+    "2d_periodic_mirror_emhd": (2, (13, 4, 1), "pm", 1, True),
+    "2d_thinner_than_ghosts": (2, (16, 2, 1), "om", 0, False),
+    "2d_above_one_launch": (2, (380, 350, 1), "pp", 0, False),
+    "2d_above_wide_solve": (2, (140, 130, 1), "op", 0, True),
+    "3d_mixed_boundaries_emhd": (3, (9, 8, 6), "omp", 1, True),
+    "3d_periodic_ideal": (3, (7, 5, 4), "ppp", 0, False),
+}
+
+
+@pytest.mark.parametrize("solver", ["fd", "mixed", "escalating"])
+@pytest.mark.parametrize("case", sorted(STEP_CASES))
+def test_time_step_equals_its_stages(torch, case, solver):
+    """grim_time_step (ghosts filled in one launch with the communicate in
+    it, the explicit half of small one- and two-dimensional grids in one
+    launch, the fold and the EMFs inside the solve, the last communicate in
+    the end of the step) against the stage-level entry points, which run each
+    piece by itself: two steps equal bit for bit, every ghost zone, time, dt,
+    right-hand side and residual mask included."""
+    from grim_amd import capi
+    from grim_amd.timestepper import TimeStepper, grid_config
+
+    dim, (N1, N2, N3), bc, recon, emhd = STEP_CASES[case]
+    code = {"p": capi.BC_PERIODIC, "o": capi.BC_OUTFLOW, "m": capi.BC_MIRROR}
+    kinds = [code[c] for c in bc.ljust(3, "p")]
+    cfg = grid_config(N1=N1, N2=N2, N3=N3, dim=dim, boundaryLeft=kinds[0], boundaryRight=kinds[0],
+                      boundaryBottom=kinds[1], boundaryTop=kinds[1], boundaryBack=kinds[2], boundaryFront=kinds[2],
+                      reconstruction=recon, riemannSolver=capi.RIEMANN_LLF, residualScaling=1 if emhd else 0,
+                      CourantFactor=0.4)
+    p = capi.default_params(emhd)
+    p.maxNonLinearIter = 6
+    opts = {"fd": None, "mixed": capi.newton_opts(capi.JAC_ANALYTIC, capi.LU_FP32),
+            "escalating": capi.newton_opts(capi.JAC_ANALYTIC, capi.LU_FP32_FP64)}[solver]
+    rng = np.random.default_rng(7)
+    n3, n2, n1 = cfg.shape
+    x = [np.arange(n) / max(n, 2) for n in (n3, n2, n1)]
+    wave = lambda k: np.sin(2 * np.pi * (k[0] * x[0][:, None, None] + k[1] * x[1][:, None] + k[2] * x[2] + rng.random()))  # noqa: E731,E501
+    prim = np.zeros((p.dof, n3, n2, n1))
+    for v in range(p.dof):
+        base = {0: 1., 1: 2., p.nf: 0.2, p.nf + 1: 0.3}.get(v, 0.)
+        prim[v] = base + 0.05 * wave((1, 2, 1)) * wave((2, 1, 1))
+    runs = []
+    for staged in (False, True):
+        ts = TimeStepper(p, cfg, opts=opts)
+        ts.primOld = prim
+        ts.set_time(0., 1e-3)
+        for _ in range(2):
+            if not staged:
+                ts.timeStep(stats=False)
+                continue
+            ts.stepBegin()
+            for st in range(2):
+                ts.foldRHS(st)
+                ts.solve(st)
+                ts.stageFinish(st)
+            ts.stepEnd()
+        it, l2 = ts.lastSolveStats()
+        R = ts.computeResidual(1, torch.from_numpy(ts.primOld).cuda()).cpu().numpy() if solver == "fd" else None
+        runs.append((ts.primOld, it, l2, ts.time, ts.dt, R))
+        ts.close()
+    a, b = runs
+    inner = tuple(slice(3, -3) if d < dim else slice(None) for d in (2, 1, 0))
+    assert np.isfinite(a[0].reshape(p.dof, *cfg.shape)[(slice(None),) + inner]).all()
+    for k in range(5):
+        np.testing.assert_array_equal(a[k], b[k])
+    if solver == "fd":  # reads the stored right-hand side and residual mask
+        np.testing.assert_array_equal(a[5], b[5])
+
+
 @pytest.mark.parametrize("solver", ["fd_fp64", "mixed_escalating"])
 def test_fast_explicit_torus_steps_match_oracle(torch, solver):
     """Two EMHD torus steps with the fast explicit stage against the oracle's
