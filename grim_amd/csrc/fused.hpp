@@ -106,25 +106,27 @@ __device__ __forceinline__ void fastClosure(double rho, double u, double p, doub
                                             double radius, FastClosure& c) {
 #pragma clang fp contract(on)
   const double cs2 = prm.gam * p * fastRcp(rho + prm.gam * u);
+  // locals, stored once below: members stored branch by branch are merged
+  // into stores at a selected address, which keeps c in scratch memory
+  double tau, chi, nu;
   if (prm.closure == GRIM_CLOSURE_LINEAR_MODES) {
-    c.tau = 1.;
-    c.chiOverTau = c.nuOverTau = cs2;
+    tau = 1.;
+    chi = nu = cs2;
   } else if (prm.closure == GRIM_CLOSURE_PER_ZONE) {
-    c.tau = prm.tau0;
-    c.chiOverTau = alphaC * cs2;
-    c.nuOverTau = alphaV * cs2;
+    tau = prm.tau0;
+    chi = alphaC * cs2;
+    nu = alphaV * cs2;
   } else if (prm.closure == GRIM_CLOSURE_SHOCK_TESTS) {
-    c.tau = 0.1;
-    c.chiOverTau = prm.condAlpha * cs2;
-    c.nuOverTau = prm.viscAlpha * cs2;
+    tau = 0.1;
+    chi = prm.condAlpha * cs2;
+    nu = prm.viscAlpha * cs2;
   } else if (prm.closure == GRIM_CLOSURE_BUOYANCY) {
-    const double chi = fastSqrt(radius);
-    c.tau = fastDiv(1.2 * chi, cs2);
-    c.chiOverTau = cs2 * (1. / 1.2);
-    c.nuOverTau = 0.;
+    tau = fastDiv(1.2 * fastSqrt(radius), cs2);
+    chi = cs2 * (1. / 1.2);
+    nu = 0.;
   } else {
     const double dyn = radius * fastSqrt(radius);
-    double tau = dyn;
+    tau = dyn;
     if constexpr (L::COND_ON) {
       const double q = prm.highOrderCond ? qTilde * T * fastSqrt(rho * prm.condAlpha * cs2) : qTilde;
       double y = fastDiv(fabs(q), prm.condClosureFactor * rho * (cs2 * fastSqrt(cs2)));
@@ -141,11 +143,13 @@ __device__ __forceinline__ void fastClosure(double rho, double u, double p, doub
       y = exp((1. - y) * 100.);
       tau = smin(tau, dyn * (fastDiv(y, y + 1.) + 1.e-5));
     }
-    c.tau = tau;
     const double maxAlpha = fastDiv(1. - cs2, 2. * cs2 + 1.e-12);
-    c.chiOverTau = smin(maxAlpha, prm.condAlpha) * cs2;
-    c.nuOverTau = smin(maxAlpha, prm.viscAlpha) * cs2;
+    chi = smin(maxAlpha, prm.condAlpha) * cs2;
+    nu = smin(maxAlpha, prm.viscAlpha) * cs2;
   }
+  c.tau = tau;
+  c.chiOverTau = chi;
+  c.nuOverTau = nu;
 }
 
 // Coefficient and old elements of the EMHD rows (elemOld's u_mu and T; the

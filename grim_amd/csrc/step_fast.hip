@@ -22,7 +22,10 @@
 // results are tested against the exact kernels and the oracle to 1e-12.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "fast_ops.hpp"
+#include "fused.hpp"
 #include "grim_hip.h"
 #include "runtime.hpp"
 #include "step_fast.hpp"
@@ -32,16 +35,16 @@
 namespace grim {
 namespace {
 
-// WENO5 face value of one zone from y[0..4] = in[i-2 .. i+2]: SIDE 0 the
-// value at i + 1/2 (grim's primRight), SIDE 1 at i - 1/2 (primLeft).
+// WENO5 face values of one zone from y[0..4] = in[i-2 .. i+2]: `right` at
+// i + 1/2 (grim's primRight), `left` at i - 1/2 (primLeft); a side that is
+// not used costs only its own candidates.
 // grim's smoothness indicators (weno5.cpp:165-193) are the quadratic forms
 // beta_k = 13/12 (second difference)^2 + 1/4 (first-difference combination)^2;
 // they are formed here as 12 beta_k (eps2 scaled with them), a factor that
 // cancels in the normalised weights.  The weights c_k / beta_k^2 and their
 // sum are scaled by beta_1^2 beta_2^2 beta_3^2 and the linear weights folded
-// into the candidate stencils, which leaves one quotient.
-template <int SIDE>
-__device__ __forceinline__ double weno5Fast(const double* y) {
+// into the candidate stencils, which leaves one quotient per side.
+__device__ __forceinline__ void weno5Fast(const double* y, double& left, double& right) {
   const double eps = 12. * 1.0e-17;
   const double y0 = y[0], y1 = y[1], y2 = y[2], y3 = y[3], y4 = y[4];
   const double a12 = fabs(y1) + fabs(y2), a23 = fabs(y2) + fabs(y3);
@@ -53,30 +56,22 @@ __device__ __forceinline__ double weno5Fast(const double* y) {
   const double beta3 = 13. * d3 * d3 + 3. * e3 * e3 + eps * (1. + a23 + fabs(y4));
   const double b1 = beta1 * beta1, b2 = beta2 * beta2, b3 = beta3 * beta3;
   const double p1 = b2 * b3, p2 = b1 * b3, p3 = b1 * b2;
-  double num, den;
-  if constexpr (SIDE == 0) {
-    // linear weights (1, 10, 5) / 16 of the candidates at i + 1/2
-    num = p1 * (0.375 * y0 - 1.25 * y1 + 1.875 * y2) + p2 * (-1.25 * y1 + 7.5 * y2 + 3.75 * y3) +
-          p3 * (1.875 * y2 + 3.75 * y3 - 0.625 * y4);
-    den = p1 + 10. * p2 + 5. * p3;
-  } else {
-    // (5, 10, 1) / 16 at i - 1/2
-    num = p1 * (-0.625 * y0 + 3.75 * y1 + 1.875 * y2) + p2 * (3.75 * y1 + 7.5 * y2 - 1.25 * y3) +
-          p3 * (1.875 * y2 - 1.25 * y3 + 0.375 * y4);
-    den = 5. * p1 + 10. * p2 + p3;
-  }
-  return fastDiv(num, den);
+  // linear weights (1, 10, 5) / 16 of the candidates at i + 1/2
+  right = fastDiv(p1 * (0.375 * y0 - 1.25 * y1 + 1.875 * y2) + p2 * (-1.25 * y1 + 7.5 * y2 + 3.75 * y3) +
+                      p3 * (1.875 * y2 + 3.75 * y3 - 0.625 * y4),
+                  p1 + 10. * p2 + 5. * p3);
+  // (5, 10, 1) / 16 at i - 1/2
+  left = fastDiv(p1 * (-0.625 * y0 + 3.75 * y1 + 1.875 * y2) + p2 * (3.75 * y1 + 7.5 * y2 - 1.25 * y3) +
+                     p3 * (1.875 * y2 - 1.25 * y3 + 0.375 * y4),
+                 5. * p1 + 10. * p2 + p3);
 }
 
-template <int RECON, int SIDE>
-__device__ __forceinline__ double faceValue(const double* y, double theta) {
-  if constexpr (RECON == GRIM_RECON_WENO5) {
-    return weno5Fast<SIDE>(y);
-  } else {
-    double l, r;
-    reconstructZone<RECON>(y, theta, l, r);
-    return SIDE ? l : r;
-  }
+template <int RECON>
+__device__ __forceinline__ void faceValues(const double* y, double theta, double& left, double& right) {
+  if constexpr (RECON == GRIM_RECON_WENO5)
+    weno5Fast(y, left, right);
+  else
+    reconstructZone<RECON>(y, theta, left, right);
 }
 
 // fluidElement::set's kinematics (physics.cpp:60-116) with one reciprocal of
@@ -225,42 +220,6 @@ __device__ __forceinline__ void fluxesFast(const double* P, const Kinematics& k,
   if constexpr (L::VISC_ON) F[L::DP] = gu * P[L::DP];
 }
 
-// computeMinMaxCharSpeeds (riemannsolver.cpp:54-200) along DIR = 0, 1, 2.
-// The unit covectors A = dX^(DIR+1), B = dt pick single inverse-metric
-// entries: A.A = g^{ss}, B.B = g^{00}, A.B = g^{s0}, A.u = u^s, B.u = u^0.
-template <class L, int DIR>
-__device__ __forceinline__ void charSpeedsFast(const Kinematics& k, const Closure& c, double gconSS, double gcon00,
-                                               double gcon0S, const DevParams& prm, double& minSpeed,
-                                               double& maxSpeed) {
-  const double rhoGu = k.rho + prm.gam * k.u;
-  const double cAlvenSqr = fastDiv(k.bSqr, rhoGu + k.bSqr);
-  double csSqr = c.soundSpeed * c.soundSpeed;
-  double cVisSqr = 0., cConSqr = 0.;
-  if constexpr (L::EMHD) {
-    const double invTau = fastRcp(c.tau);
-    if constexpr (L::VISC_ON) cVisSqr = fastDiv((4. / 3.) * k.rho * c.nu * invTau, rhoGu);
-    if constexpr (L::COND_ON) cConSqr = (prm.gam - 1.) * c.chi * invTau;
-  }
-  cConSqr = 0.5 * (csSqr + cConSqr + sqrt(csSqr * csSqr + cConSqr * cConSqr));
-  csSqr = cConSqr + cVisSqr;
-  csSqr = csSqr + cAlvenSqr - csSqr * cAlvenSqr;
-  csSqr = csSqr > 1. ? 1. : csSqr;
-  constexpr int sdir = DIR + 1;
-  const double ASqr = gconSS, BSqr = gcon00, ADotB = gcon0S;
-  const double ADotU = k.uCon[sdir], BDotU = k.uCon[0];
-  const double A = (BDotU * BDotU) - (BSqr + BDotU * BDotU) * csSqr;
-  const double B = 2. * (ADotU * BDotU - (ADotB + ADotU * BDotU) * csSqr);
-  const double C = ADotU * ADotU - (ASqr + ADotU * ADotU) * csSqr;
-  const double discr = sqrt(smax(B * B - 4. * A * C, 1.e-16));
-  const double inv2A = 0.5 * fastRcp(A);
-  double mn = (B - discr) * inv2A;
-  double mx = (B + discr) * inv2A;
-  mn = mn > -1.e-15 ? -1.e-15 : mn;
-  mx = mx < 1.e-15 ? 1.e-15 : mx;
-  minSpeed = mn;
-  maxSpeed = mx;
-}
-
 // The geometry one side of a face needs: the zone geometry, the inverse
 // metric entry g^{ss} of the face direction and r (the torus closure).
 struct FaceGeom {
@@ -282,92 +241,356 @@ __device__ __forceinline__ void loadFaceGeom(const double* geom, int64_t n, uint
   G.r = ldOff(geom + LOC_R * n, zb);
 }
 
-// One side of a face (as faceState in step.hip): the face value of every
-// variable, the element at the face geometry, its flux, conserved
-// variables and speeds.  zb: the byte offset of the face's zone in a plane,
-// zgb: that of its (X1, X2) column in a geometry plane.
-template <class L, int DIR, int RECON, int SIDE>
-__device__ __forceinline__ void faceStateFast(const StepArgs& a, uint32_t zb, uint32_t zgb,
-                                              const double* __restrict__ prim,
-                                              const double* __restrict__ geomFace, double (&F)[L::DOF],
-                                              double (&U)[L::DOF], double& mn, double& mx) {
-  const int64_t n = a.D.n;
-  // the stencil's offsets along DIR, shared by every variable's plane
-  uint32_t off[5];
+// The element of one face value (fluidElement::set, physics.cpp:53-183), its
+// computeFluxes(DIR + 1) and computeFluxes(0) (:185-217) and its speeds along
+// DIR (computeMinMaxCharSpeeds, riemannsolver.cpp:54-200).
+//
+// In the identity form of the solve's residual (fused.hpp): lowered spatial
+// vectors from gamma_ij, b_mu = (B_mu + b^0 u_mu)/u^0, and the two rows of
+// T^mu_nu as A^mu u_nu + C^mu b_nu + d^mu_nu E, so no other contravariant
+// component is formed.  The conserved field is g (b^i u^0 - b^0 u^i) = g B^i,
+// its flux g (B^c u^d - B^d u^c)/u^0.  The speeds read chi/tau and nu/tau,
+// in which tau cancels: the torus closure's two exponentials do not enter
+// the fluxes.  The unit covectors of the speeds pick single entries of the
+// inverse metric.  (Against the reference's order of operations this took
+// the two states of a face from 2,750 to about 1,600 VALU instructions.)
+//
+// The results go to `out` one by one, first the speeds, out.speeds(mn, mx),
+// then out.row(v, F_v, U_v) without the common factor g: a consumer that
+// combines each row at once never holds all of them.
+template <class L, int DIR, class Out>
+__device__ __forceinline__ void faceElement(const double* P, const FaceGeom& fg, const DevParams& prm, Out&& out) {
+  constexpr int D = DIR + 1;
+  const ZoneGeom& G = fg.zg;
+  const double rho = smax(P[RHO], prm.rhoFloor), u = smax(P[UU], prm.uFloor);
+  const double *ut = P + U1, *B = P + L::B1;
+  const double p = (prm.gam - 1.) * u;
+  double utLow[3], BLow[3];
+  lower3(G, ut, utLow);
+  lower3(G, B, BLow);
+  const double lor = fastSqrt(1. + dot3(ut, utLow));
+  const double u0 = fastDiv(lor, G.alpha), invU0 = fastDiv(G.alpha, lor), ga = lor * G.alpha;
+  double uc[3];  // u^1..u^3
 #pragma unroll
-  for (int q = 0; q < 5; q++) off[q] = zb + (uint32_t)((q - 3 + SIDE) * a.D.s[DIR] * 8);
-  double P[L::DOF];
+  for (int i = 0; i < 3; i++) uc[i] = ut[i] - ga * G.gcon0[i + 1];
+  const double ud = uc[DIR];
+  double uCov[4], bCov[4];
+  uCov[0] = G.cov(0, 1) * ut[0] + G.cov(0, 2) * ut[1] + G.cov(0, 3) * ut[2] - G.alpha * lor;
+  const double b0 = dot3(B, utLow), bd = (B[DIR] + b0 * ud) * invU0;
+  bCov[0] = (G.cov(0, 1) * B[0] + G.cov(0, 2) * B[1] + G.cov(0, 3) * B[2] + b0 * uCov[0]) * invU0;
 #pragma unroll
-  for (int v = 0; v < L::DOF; v++) {
-    double y[5];
-#pragma unroll
-    for (int q = 0; q < 5; q++) y[q] = ldOff(prim + v * n, off[q]);
-    P[v] = faceValue<RECON, SIDE>(y, a.theta);
+  for (int i = 0; i < 3; i++) {
+    uCov[i + 1] = utLow[i];
+    bCov[i + 1] = (BLow[i] + b0 * utLow[i]) * invU0;
   }
-  FaceGeom G;
-  loadFaceGeom<DIR>(geomFace, a.D.ng, zgb, G);
-  Kinematics kk;
-  Closure cc;
-  kinematicsFast<L>(P, G.zg, a.prm, kk);
-  closureFast<L>(P, kk, a.prm, G.r, cc);
-  const StressInv si = stressInv<L>(kk, cc);
-  fluxesFast<L, DIR + 1>(P, kk, cc, si, G.zg.g, F);
-  fluxesFast<L, 0>(P, kk, cc, si, G.zg.g, U);
-  charSpeedsFast<L, DIR>(kk, cc, G.gconSS, G.zg.gcon0[0], G.zg.gcon0[DIR + 1], a.prm, mn, mx);
+  const double bsq = (dot3(B, BLow) + b0 * b0) * invU0 * invU0 + prm.bSqrFloor;
+  const double rhoGu = rho + prm.gam * u, invRhoGu = fastRcp(rhoGu);
+  const double cs2 = prm.gam * p * invRhoGu;
+  const double w = rho + u + p + bsq;
+  double Ad = w * ud, A0 = w * u0, Cd = -bd, C0 = -b0, E = p + 0.5 * bsq;
+  double conSqr = 0., visSqr = 0.;
+  if constexpr (L::EMHD) {
+    const double T = smax(p * fastRcp(rho), prm.tFloor), ib = fastRsqrt(bsq);
+    FastClosure cl;
+    fastClosure<L>(rho, u, p, T, bsq, 0., 0., prm, 1., 1., fg.r, cl);
+    if constexpr (L::COND_ON) {
+      const double qb = (prm.highOrderCond ? P[L::Q] * T * fastSqrt(rho * prm.condAlpha * cs2) : P[L::Q]) * ib;
+      Ad = Ad + qb * bd;
+      A0 = A0 + qb * b0;
+      Cd = Cd + qb * ud;
+      C0 = C0 + qb * u0;
+      conSqr = (prm.gam - 1.) * cl.chiOverTau;
+    }
+    if constexpr (L::VISC_ON) {
+      const double dP = prm.highOrderVisc ? P[L::DP] * fastSqrt(T * rho * prm.viscAlpha * cs2) : P[L::DP];
+      const double third = dP * (1. / 3.), dPb = dP * ib * ib;
+      Ad = Ad + third * ud;
+      A0 = A0 + third * u0;
+      Cd = Cd - dPb * bd;
+      C0 = C0 - dPb * b0;
+      E = E + third;
+      visSqr = (4. / 3.) * rho * cl.nuOverTau * invRhoGu;
+    }
+  }
+  {
+    const double alfSqr = bsq * fastRcp(rhoGu + bsq);
+    double cSqr = 0.5 * (cs2 + conSqr + fastSqrt(cs2 * cs2 + conSqr * conSqr)) + visSqr;
+    cSqr = cSqr + alfSqr - cSqr * alfSqr;
+    cSqr = cSqr > 1. ? 1. : cSqr;
+    const double A = u0 * u0 - (G.gcon0[0] + u0 * u0) * cSqr;
+    const double Bq = 2. * (ud * u0 - (G.gcon0[D] + ud * u0) * cSqr);
+    const double C = ud * ud - (fg.gconSS + ud * ud) * cSqr;
+    const double discr = fastSqrt(smax(Bq * Bq - 4. * A * C, 1.e-16));
+    const double inv2A = 0.5 * fastRcp(A);
+    const double mn = (Bq - discr) * inv2A, mx = (Bq + discr) * inv2A;
+    out.speeds(mn > -1.e-15 ? -1.e-15 : mn, mx < 1.e-15 ? 1.e-15 : mx);
+  }
+  const double Frho = rho * ud, Urho = rho * u0;
+  out.row(RHO, Frho, Urho);
+  out.row(UU, Ad * uCov[0] + Cd * bCov[0] + Frho, A0 * uCov[0] + C0 * bCov[0] + E + Urho);
+#pragma unroll
+  for (int nu = 1; nu < 4; nu++)
+    out.row(UU + nu, Ad * uCov[nu] + Cd * bCov[nu] + (nu == D ? E : 0.), A0 * uCov[nu] + C0 * bCov[nu]);
+  if constexpr (L::COND_ON) out.row(L::Q, ud * P[L::Q], u0 * P[L::Q]);
+  if constexpr (L::VISC_ON) out.row(L::DP, ud * P[L::DP], u0 * P[L::DP]);
+#pragma unroll
+  for (int c = 0; c < 3; c++)
+    out.row(L::B1 + c, c == DIR ? 0. : (B[c] * ud - B[DIR] * uc[c]) * invU0, B[c]);
 }
 
-// The split face kernel of step.hip with the fast element: wavefronts 0-1
-// the left states, 2-3 the right states, which meet in LDS.
+// A face's left state in LDS, each entry a row over the workgroup's lanes:
+// the conserved variables, the two speeds and the fluxes but that of the
+// field along DIR, which is zero.
+template <class L, int LANES>
+using FaceSlots = double[2 * L::DOF + 1][LANES];
+
+// Row of flux v, and whether it has one.
+template <class L, int DIR>
+__device__ __forceinline__ int fluxSlot(int v) {
+  return L::DOF + 2 + (v > L::B1 + DIR ? v - 1 : v);
+}
+template <class L, int DIR>
+__device__ __forceinline__ bool noFlux(int v) {
+  return v == L::B1 + DIR;
+}
+
+template <class L, int DIR, int LANES>
+struct StoreSide {
+  FaceSlots<L, LANES>& sh;
+  int slot;
+  __device__ __forceinline__ void speeds(double mn, double mx) {
+    sh[L::DOF][slot] = mn;
+    sh[L::DOF + 1][slot] = mx;
+  }
+  __device__ __forceinline__ void row(int v, double F, double U) {
+    sh[v][slot] = U;
+    if (!noFlux<L, DIR>(v)) sh[fluxSlot<L, DIR>(v)][slot] = F;
+  }
+};
+
+// The right state of a face on its way out of faceElement: the HLL or LLF
+// flux of each row against the left state in LDS (riemannsolver.cpp:270-328),
+// stored at byte offset zb of its flux plane.
+template <class L, int DIR, int LANES>
+struct SolveFace {
+  const StepArgs& a;
+  FaceSlots<L, LANES>& sh;
+  int slot;
+  double metric;
+  double* flux;
+  uint32_t zb;
+  double mn, mx, k, b;  // speeds; HLL: g/(mx - mn) and mn mx, LLF: g/2 and the largest speed
+  __device__ __forceinline__ void speeds(double mnR, double mxR) {
+    mn = stdmin(sh[L::DOF][slot], mnR);
+    mx = stdmax(sh[L::DOF + 1][slot], mxR);
+    const bool hll = a.riemann == GRIM_RIEMANN_HLL;
+    k = hll ? metric * fastRcp(mx - mn) : 0.5 * metric;
+    b = hll ? mn * mx : stdmax(mx, -mn);
+  }
+  __device__ __forceinline__ void row(int v, double FR, double UR) {
+    const double FL = noFlux<L, DIR>(v) ? 0. : sh[fluxSlot<L, DIR>(v)][slot], UL = sh[v][slot];
+    const double f = a.riemann == GRIM_RIEMANN_HLL ? mx * FL - mn * FR + b * (UR - UL) : FL + FR - b * (UR - UL);
+    stOff(flux + v * a.D.n, zb, f * k);
+  }
+};
+
+// A state held in registers until its partner is in LDS.
+template <class L>
+struct HoldSide {
+  double F[L::DOF], U[L::DOF], mn, mx;
+  __device__ __forceinline__ void speeds(double a, double b) {
+    mn = a;
+    mx = b;
+  }
+  __device__ __forceinline__ void row(int v, double f, double u) {
+    F[v] = f;
+    U[v] = u;
+  }
+  template <class Out>
+  __device__ __forceinline__ void to(Out&& out) const {
+    out.speeds(mn, mx);
+#pragma unroll
+    for (int v = 0; v < L::DOF; v++) out.row(v, F[v], U[v]);
+  }
+};
+
+// The face values of every variable of the zone at byte offset zb.
+template <class L, int DIR, int RECON>
+__device__ __forceinline__ void reconstructBoth(const StepArgs& a, const double* __restrict__ prim, uint32_t zb,
+                                                double* left, double* right) {
+  const int64_t n = a.D.n;
+  uint32_t off[5];
+#pragma unroll
+  for (int q = 0; q < 5; q++) off[q] = zb + (uint32_t)((q - 2) * a.D.s[DIR] * 8);
+  // Two variables' stencils are in flight while the two before them are
+  // reconstructed; pinning each result keeps the compiler from issuing every
+  // variable's loads first, which would hold 50 values in registers.
+  constexpr int GROUP = 2, GROUPS = (L::DOF + GROUP - 1) / GROUP;
+  double y[2][GROUP][5];
+  auto load = [&](int g) {
+#pragma unroll
+    for (int e = 0; e < GROUP; e++)
+#pragma unroll
+      for (int q = 0; q < 5; q++)
+        if (g * GROUP + e < L::DOF) y[g & 1][e][q] = ldOff(prim + (g * GROUP + e) * n, off[q]);
+  };
+  load(0);
+#pragma unroll
+  for (int g = 0; g < GROUPS; g++) {
+    if (g + 1 < GROUPS) load(g + 1);
+#pragma unroll
+    for (int e = 0; e < GROUP; e++) {
+      const int v = g * GROUP + e;
+      if (v >= L::DOF) continue;
+      faceValues<RECON>(y[g & 1][e], a.theta, left[v], right[v]);
+      asm volatile("" : "+v"(left[v]), "+v"(right[v]));
+    }
+  }
+}
+
+// X1 faces of large grids.  A lane takes one zone: both its face values from
+// one set of smoothness indicators, then the elements of both.  The state it
+// leaves right of itself is the next lane's left state, read from LDS within
+// the wavefront (no barrier), so no state is built twice.  The zones of all
+// rows (one more than the faces of a row) are numbered through; a wavefront
+// takes 63 of them and the one before.  Bound by FP64 issue (1,660
+// instructions per zone, about 210 us of 350 at 192x192x128 zones, EMHD; 510
+// with two threads per face) and by the 780 MB it moves; a fourth wavefront
+// per SIMD (blocks of 64) adds nothing.
+constexpr int kRowBlock = 128;
+template <class L, int RECON>
+__global__ __launch_bounds__(kRowBlock) __attribute__((amdgpu_waves_per_eu(3))) void faceFluxRowKernel(
+    StepArgs a, Box box, const double* __restrict__ prim, const double* __restrict__ geomFace,
+    double* __restrict__ flux) {
+  __shared__ FaceSlots<L, kRowBlock> sh;
+  const int lane = threadIdx.x & 63;
+  const unsigned wave = blockIdx.x * (kRowBlock / 64) + (threadIdx.x >> 6);
+  const unsigned rowZones = (unsigned)(box.hi[0] - box.lo[0]) + 1u, rows1 = (unsigned)(box.hi[1] - box.lo[1]);
+  const unsigned total = rowZones * rows1 * (unsigned)(box.hi[2] - box.lo[2]);
+  const unsigned t = wave * 63u + (unsigned)lane;
+  if (t >= total) return;
+  const unsigned row = t / rowZones, iz = t % rowZones;
+  const uint32_t i = (uint32_t)box.lo[0] - 1u + iz;
+  const uint32_t zgb = (i + (uint32_t)(box.lo[1] + (int)(row % rows1)) * (uint32_t)a.D.s[1]) * 8u;
+  const uint32_t zb = zgb + (uint32_t)(box.lo[2] + (int)(row / rows1)) * (uint32_t)a.D.s[2] * 8u;
+  double left[L::DOF], right[L::DOF];
+  reconstructBoth<L, 0, RECON>(a, prim, zb, left, right);
+  FaceGeom G;
+  loadFaceGeom<0>(geomFace, a.D.ng, zgb + 8u, G);  // the face right of the zone
+  faceElement<L, 0>(right, G, a.prm, StoreSide<L, 0, kRowBlock>{sh, (int)threadIdx.x});
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  if (lane == 0 || iz == 0) return;
+  loadFaceGeom<0>(geomFace, a.D.ng, zgb, G);
+  faceElement<L, 0>(left, G, a.prm, SolveFace<L, 0, kRowBlock>{a, sh, (int)threadIdx.x - 1, G.zg.g, flux, zb});
+}
+
+// X2 and X3 faces of large grids.  A lane walks `steps` faces along DIR in
+// one (X1, other) column with the five stencil values of every variable in
+// registers, so each primitive is loaded once per walk (and four more at its
+// start), one zone ahead of its use; it keeps the state right of the zone it
+// has just left (in its own LDS slots) for the next face, so each zone's
+// indicators and elements are formed once.  That takes 224 registers, two
+// wavefronts per SIMD; loading the stencils again for every zone leaves room
+// for three but reads each value five times, mostly past the L2 (a lane's
+// column is its own): 482 and 553 us for X2 and X3 of 192x192x128 EMHD zones
+// against 377 and 382 (510 and 525 with two threads per face).  Bound by FP64
+// issue as the X1 kernel.
+template <class L, int DIR, int RECON>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void faceFluxMarchKernel(
+    StepArgs a, Box box, int steps, const double* __restrict__ prim, const double* __restrict__ geomFace,
+    double* __restrict__ flux) {
+  __shared__ FaceSlots<L, kBlock> sh;
+  constexpr int OTHER = 3 - DIR;
+  const int64_t n = a.D.n;
+  const unsigned ni = (unsigned)(box.hi[0] - box.lo[0]);
+  const unsigned cols = ni * (unsigned)(box.hi[OTHER] - box.lo[OTHER]);
+  const unsigned perSeg = (cols + kBlock - 1) / kBlock;
+  const unsigned seg = blockIdx.x / perSeg;
+  const unsigned c = (blockIdx.x % perSeg) * kBlock + threadIdx.x;
+  if (c >= cols) return;
+  const int slot = (int)threadIdx.x;
+  const int first = box.lo[DIR] + (int)seg * steps;
+  const int last = min(first + steps, box.hi[DIR]);  // faces [first, last)
+  const uint32_t sB = (uint32_t)a.D.s[DIR] * 8u;
+  // bytes from one face to the next in a geometry plane (X3: the same column)
+  const uint32_t gB = DIR == 1 ? sB : 0u;
+  const uint32_t other = (uint32_t)(box.lo[OTHER] + (int)(c / ni));
+  uint32_t zgb = ((uint32_t)box.lo[0] + c % ni) * 8u + (DIR == 1 ? (uint32_t)first * sB : other * (uint32_t)a.D.s[1] * 8u);
+  uint32_t zb = ((uint32_t)box.lo[0] + c % ni) * 8u + other * (uint32_t)a.D.s[OTHER] * 8u + (uint32_t)first * sB;
+  // the zone before the first face, then each zone of the walk: its left
+  // state closes a face, its right state opens the next
+  double y[L::DOF][5];
+  zb -= sB;
+#pragma unroll
+  for (int v = 0; v < L::DOF; v++)
+#pragma unroll
+    for (int q = 0; q < 5; q++) y[v][q] = ldOff(prim + v * n, zb + (uint32_t)((q - 2) * a.D.s[DIR] * 8));
+  for (int f = first - 1; f < last; f++) {
+    const bool more = f + 1 < last;
+    double next[L::DOF], left[L::DOF], right[L::DOF];
+    if (more) {
+#pragma unroll
+      for (int v = 0; v < L::DOF; v++) next[v] = ldOff(prim + v * n, zb + 3 * sB);
+    }
+    FaceGeom G;
+    if (f >= first) loadFaceGeom<DIR>(geomFace, a.D.ng, zgb, G);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int v = 0; v < L::DOF; v++) {
+      faceValues<RECON>(y[v], a.theta, left[v], right[v]);
+      asm volatile("" : "+v"(left[v]), "+v"(right[v]));
+    }
+    if (f >= first) {
+      faceElement<L, DIR>(left, G, a.prm, SolveFace<L, DIR, kBlock>{a, sh, slot, G.zg.g, flux, zb});
+      zgb += gB;
+    }
+    if (more) {
+      loadFaceGeom<DIR>(geomFace, a.D.ng, zgb, G);
+      faceElement<L, DIR>(right, G, a.prm, StoreSide<L, DIR, kBlock>{sh, slot});
+#pragma unroll
+      for (int v = 0; v < L::DOF; v++) {
+#pragma unroll
+        for (int q = 0; q < 4; q++) y[v][q] = y[v][q + 1];
+        y[v][4] = next[v];
+      }
+    }
+    zb += sB;
+  }
+}
+
+// Small grids: two threads per face, wavefronts 0-1 of a workgroup the left
+// states, 2-3 the right states, which meet in LDS (as the split face kernel of
+// step.hip): twice the wavefronts, each half as long.
 template <class L, int DIR, int RECON>
 __global__ __launch_bounds__(kBlock) void faceFluxFastKernel(StepArgs a, Box box, const double* __restrict__ prim,
                                                              const double* __restrict__ geomFace,
                                                              double* __restrict__ flux) {
-  __shared__ double sh[2 * L::DOF + 2][kFacesPerBlock];
+  __shared__ FaceSlots<L, kFacesPerBlock> sh;
   const int side = threadIdx.x / kFacesPerBlock;
   const int lf = threadIdx.x % kFacesPerBlock;
   const int64_t f = (int64_t)blockIdx.x * kFacesPerBlock + lf;
   const bool active = f < box.count();
-  const int64_t n = a.D.n;
   uint32_t zb = 0;
-  double F[L::DOF], U[L::DOF], mn = 0., mx = 0.;
+  double P[L::DOF], unused[L::DOF];
+  FaceGeom G;
   if (active) {
     int i, j, k;
     box.at(f, i, j, k);
     const uint32_t zgb = ((uint32_t)i + (uint32_t)j * (uint32_t)a.D.s[1]) * 8u;
     zb = zgb + (uint32_t)k * (uint32_t)a.D.s[2] * 8u;
-    if (side == 0) {
-      faceStateFast<L, DIR, RECON, 0>(a, zb, zgb, prim, geomFace, F, U, mn, mx);
-    } else {
-      faceStateFast<L, DIR, RECON, 1>(a, zb, zgb, prim, geomFace, F, U, mn, mx);
-#pragma unroll
-      for (int v = 0; v < L::DOF; v++) {
-        sh[v][lf] = F[v];
-        sh[L::DOF + v][lf] = U[v];
-      }
-      sh[2 * L::DOF][lf] = mn;
-      sh[2 * L::DOF + 1][lf] = mx;
-    }
+    if (side == 0)
+      reconstructBoth<L, DIR, RECON>(a, prim, zb - (uint32_t)a.D.s[DIR] * 8u, unused, P);
+    else
+      reconstructBoth<L, DIR, RECON>(a, prim, zb, P, unused);
+    loadFaceGeom<DIR>(geomFace, a.D.ng, zgb, G);
+  }
+  HoldSide<L> s;
+  if (active) {
+    faceElement<L, DIR>(P, G, a.prm, s);
+    if (side == 0) s.to(StoreSide<L, DIR, kFacesPerBlock>{sh, lf});
   }
   __syncthreads();
-  if (!active || side != 0) return;
-  const double minSpeed = stdmin(mn, sh[2 * L::DOF][lf]);
-  const double maxSpeed = stdmax(mx, sh[2 * L::DOF + 1][lf]);
-  if (a.riemann == GRIM_RIEMANN_HLL) {
-    const double inv = fastRcp(maxSpeed - minSpeed);
-    const double mm = minSpeed * maxSpeed;
-#pragma unroll
-    for (int v = 0; v < L::DOF; v++) {
-      const double FR = sh[v][lf], UR = sh[L::DOF + v][lf];
-      stOff(flux + v * n, zb, (maxSpeed * F[v] - minSpeed * FR + mm * (UR - U[v])) * inv);
-    }
-  } else {
-    const double c = stdmax(maxSpeed, -minSpeed);
-#pragma unroll
-    for (int v = 0; v < L::DOF; v++) {
-      const double FR = sh[v][lf], UR = sh[L::DOF + v][lf];
-      stOff(flux + v * n, zb, 0.5 * (F[v] + FR - c * (UR - U[v])));
-    }
-  }
+  if (active && side == 1) s.to(SolveFace<L, DIR, kFacesPerBlock>{a, sh, lf, G.zg.g, flux, zb});
 }
 
 __host__ __device__ constexpr int sym4(int k, int m) {
@@ -551,26 +774,55 @@ inline unsigned blocks(int64_t count, int per) { return (unsigned)((count + per 
 
 }  // namespace
 
+// Faces from which X1's fluxes go by rows of zones, and X2's and X3's by walks,
+// instead of two threads per face.  EMHD, WENO5, both kernels, us per call:
+//   faces           32,768  110,592  262,144  512,000  884,736  1.6 M  4.7 M
+//   X1 split          13.3     24.8     43.5     74.4      117    225    612
+//   X1 rows           13.9     21.5     36.2     57.9       88    166    482
+//   X2 split          13.4     24.9     47.4     82.3      126    218    643
+//   X2 walks          28.2     32.8     53.8     80.1      110    181    461
+// (X3 as X2; with 110 us of other work in the last column).  A walk is a serial
+// chain of its faces: below half a million faces too few are in flight.
+constexpr int64_t kRowFaces = 1 << 16;
+constexpr int64_t kMarchFaces = 1 << 19;
+// Wavefronts that a launch of walks should keep: two fit a SIMD at a time, so
+// this is four rounds of the chip; fewer and longer walks (6144) are no faster.
+constexpr int64_t kMarchWaves = 8192;
+
 int launchFaceFast(const grim_params& p, const StepArgs& a, int dir, int recon, const Box& b, const double* prim,
                    const double* geomFace, double* flux, hipStream_t s) {
   GRIM_REQUIRE(planeOffsetsFit(a.D.n), "fast explicit stage: planes must hold fewer than 2^29 zones");
-  const unsigned nb = blocks(b.count(), kFacesPerBlock);
+  const int64_t faces = b.count();
+  // zones one face before the box belong to the grid (the stencil reaches two
+  // further), so a walk may start from them
+  const bool large = faces >= (dir == 0 ? kRowFaces : kMarchFaces);
   return dispatchLayout(p, [&]<class L>() -> int {
-    auto go = [&]<int DIR>() {
-      switch (recon) {
-        case GRIM_RECON_WENO5:
-          faceFluxFastKernel<L, DIR, GRIM_RECON_WENO5><<<nb, kBlock, 0, s>>>(a, b, prim, geomFace, flux);
-          break;
-        case GRIM_RECON_PPM:
-          faceFluxFastKernel<L, DIR, GRIM_RECON_PPM><<<nb, kBlock, 0, s>>>(a, b, prim, geomFace, flux);
-          break;
-        default:
-          faceFluxFastKernel<L, DIR, GRIM_RECON_MINMOD><<<nb, kBlock, 0, s>>>(a, b, prim, geomFace, flux);
+    auto go = [&]<int DIR, int RECON>() {
+      if (!large) {
+        faceFluxFastKernel<L, DIR, RECON><<<blocks(faces, kFacesPerBlock), kBlock, 0, s>>>(a, b, prim, geomFace, flux);
+      } else if constexpr (DIR == 0) {
+        const int64_t rows = (int64_t)(b.hi[1] - b.lo[1]) * (b.hi[2] - b.lo[2]);
+        const int64_t waves = (rows * (b.hi[0] - b.lo[0] + 1) + 62) / 63;
+        faceFluxRowKernel<L, RECON><<<blocks(waves, kRowBlock / 64), kRowBlock, 0, s>>>(a, b, prim, geomFace, flux);
+      } else {
+        const int len = b.hi[DIR] - b.lo[DIR];
+        const int64_t cols = faces / len;
+        int64_t steps = cols * len / (kMarchWaves * 64);
+        steps = std::max<int64_t>(4, std::min<int64_t>(16, steps));
+        const int segs = (int)((len + steps - 1) / steps);
+        const int even = (len + segs - 1) / segs;  // the walks of a column of like length
+        const unsigned nb = blocks(cols, kBlock) * (unsigned)((len + even - 1) / even);
+        faceFluxMarchKernel<L, DIR, RECON><<<nb, kBlock, 0, s>>>(a, b, even, prim, geomFace, flux);
       }
     };
-    if (dir == 0) go.template operator()<0>();
-    else if (dir == 1) go.template operator()<1>();
-    else go.template operator()<2>();
+    auto byRecon = [&]<int DIR>() {
+      if (recon == GRIM_RECON_WENO5) go.template operator()<DIR, GRIM_RECON_WENO5>();
+      else if (recon == GRIM_RECON_PPM) go.template operator()<DIR, GRIM_RECON_PPM>();
+      else go.template operator()<DIR, GRIM_RECON_MINMOD>();
+    };
+    if (dir == 0) byRecon.template operator()<0>();
+    else if (dir == 1) byRecon.template operator()<1>();
+    else byRecon.template operator()<2>();
     return checkLaunch("face fluxes (fast)");
   });
 }

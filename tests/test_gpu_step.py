@@ -423,7 +423,7 @@ def test_mixed_newton_step_close_to_fd(torch):
 # ---------------------------------------------------------------------------
 # Torus problem
 # ---------------------------------------------------------------------------
-def torus_case(emhd, N1=96, N2=48, N3=4, opts=None, scaling=1, fast=0, **pkw):
+def torus_case(emhd, N1=96, N2=48, N3=4, opts=None, scaling=1, fast=0, cfg_over=(), **pkw):
     from grim_amd import capi
 
     a = 0.9375
@@ -433,6 +433,7 @@ def torus_case(emhd, N1=96, N2=48, N3=4, opts=None, scaling=1, fast=0, **pkw):
                DoCylindrify=1, X1cyl=np.log(4 * Rin), X2cyl=1. / N2, boundaryLeft=1, boundaryRight=1,
                boundaryBottom=2, boundaryTop=2, boundaryBack=0, boundaryFront=0, reconstruction=1,
                riemannSolver=1, residualScaling=scaling, explicitFast=fast)
+    cfg.update(cfg_over)
     ts, g, p, po = make(cfg, emhd=emhd, closure=2, opts=opts, adiabaticIndex=5. / 3, **pkw)
     gm = oracle_geometry(ts, g)
     ts.initTorus(capi.torus_params())
@@ -832,6 +833,31 @@ def test_fast_explicit_pieces_match_exact(torch, emhd):
     assert err.max() < 1e-10
     ts0.close()
     ts1.close()
+
+
+@pytest.mark.parametrize("emhd,recon,riemann", [(True, 1, 1), (True, 0, 0), (False, 1, 0), (False, 2, 1)])
+def test_fast_face_fluxes_of_large_grids(torch, emhd, recon, riemann):
+    """The face kernels of large grids (a row of zones per wavefront in X1,
+    walks along X2 and X3) on a grid of odd sizes just above the 2^19 faces
+    the walks start at: rows that straddle wavefronts, walks with a remainder.
+    Against the exact stage's fluxes within the bound of the small-grid
+    kernels (both build a face value from the same stencil and an element
+    from one face value, so the rounding does not depend on the size)."""
+    kw = dict(N1=101, N2=83, N3=67, cfg_over=dict(reconstruction=recon, riemannSolver=riemann))
+    exact, g = torus_case(emhd, **kw)[:2]
+    fast = torus_case(emhd, fast=1, **kw)[0]
+    rng = np.random.default_rng(5)
+    prim = exact.primOld
+    prim[2:5] *= 1 + 0.2 * rng.standard_normal((3, g.n))
+    if emhd:
+        prim[5:7] = 1e-3 * rng.standard_normal((2, g.n)) * prim[1]
+    P = dev(torch, prim)
+    for d in range(3):
+        err, ok = scaled_diff(fast.riemannFlux(P, d).cpu().numpy(), exact.riemannFlux(P, d).cpu().numpy())
+        print(f"face fluxes dir {d}: max scaled difference {err.max():.2e} over {ok.sum()} faces", flush=True)
+        assert ok.sum() > 0.5 * g.n and err.max() < 1e-12, (d, err)
+    exact.close()
+    fast.close()
 
 
 @pytest.mark.parametrize("fast", [0, 1], ids=["exact", "fast_explicit"])
