@@ -114,7 +114,10 @@ __device__ __forceinline__ double divergence(const Dims& D, const double* dX,
 //   rhs = consOld - dt'((divF + S_expl) + 1/2 S_implOld)       (fluid rows)
 //   B   = (consOld_B - dt' divF_B) / g                        (field rows)
 // and rmax = max |rhs| (the residual scale is 1/rmax).
-template <class L, int DIM>
+// SPARSE_IMP: only the q and deltaP rows of S_implOld are read, the others
+// being zero (the grid step's own sources; a caller of the stage entry points
+// may have put other values there).
+template <class L, int DIM, bool SPARSE_IMP = false>
 __device__ __forceinline__ void foldZone(const Dims& D, const double* dX, const double* __restrict__ F,
                                          const double* __restrict__ emf, const double* __restrict__ geomC,
                                          const double* __restrict__ consOld, const double* __restrict__ sExp,
@@ -128,7 +131,8 @@ __device__ __forceinline__ void foldZone(const Dims& D, const double* dX, const 
     const double div = divergence<L, DIM>(D, dX, F, emf, v, z, i, j, filter);
     const double U = consOld[v * n + z];
     if (v < L::NF) {
-      const double si = L::EMHD ? sImp[v * n + z] : 0.;
+      const bool imp = SPARSE_IMP ? (L::VISC_ON && v == L::DP) || (L::COND_ON && v == L::Q) : L::EMHD;
+      const double si = imp ? sImp[v * n + z] : 0.;
       const double r = U - dtPrime * ((div + sExp[v * n + z]) + 0.5 * si);
       rhs[v] = r;
       rmax = stdmax(rmax, fabs(r));

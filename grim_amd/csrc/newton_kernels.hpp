@@ -505,7 +505,7 @@ __device__ __forceinline__ bool foldForSolve(const grim_zone_batch& b, const Fol
   B[0] = B[1] = B[2] = 0.;
   if (bulk) {
     double rmax;
-    foldZone<L, DIM>(f.D, f.dX, f.F, f.emf, f.geomC, f.consOld, f.sExp, f.sImp, batchDt(b), z, i, j,
+    foldZone<L, DIM, true>(f.D, f.dX, f.F, f.emf, f.geomC, f.consOld, f.sExp, f.sImp, batchDt(b), z, i, j,
                      f.fluxFilter, rhs, B, rmax);
     mask = f.scaling ? 1. / rmax : f.mask[z];
     if (lead) {

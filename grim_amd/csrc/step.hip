@@ -1852,13 +1852,13 @@ int fluxesAndEmf(grim_ctx* x, const double* prim, bool allFaces) {
 
 template <class L>
 int explicitSources(grim_ctx* x, const double* prim, const double* primOld, double* sExp, double* sImp,
-                    double* consOld) {
+                    double* consOld, bool sparseImp = false) {
   const Box b = bulkBox(x->D);
   if constexpr (L::EMHD)
     uTKernel<L><<<blocksFor(x->D.n), kBlock, 0, x->s>>>(x->a, prim, x->geomC, x->uT);
   if (x->c.explicitFast)
     return launchSourcesFast(x->p, x->a, x->c.reconstruction, b, prim, primOld, x->geomC, x->gamma40, x->uT, sExp,
-                             sImp, consOld, x->s);
+                             sImp, consOld, sparseImp, x->s);
   const unsigned nb = blocksFor(b.count());
   switch (x->c.reconstruction) {
     case GRIM_RECON_WENO5:
@@ -2192,7 +2192,7 @@ int stagePrepare(grim_ctx* x, int st, bool guessInSolve = false, bool foldInSolv
   }
   if (oneLaunch) return explicitStage<L>(x, st, primStage, reduceDt);
   if (int rc = explicitSources<L>(x, primStage, x->primOld, x->sExp, L::EMHD ? x->sImp : nullptr,
-                                  st == 0 ? x->consOld : nullptr))
+                                  st == 0 ? x->consOld : nullptr, foldInSolve))
     return rc;
   if (int rc = fluxesAndEmf<L>(x, primStage, false)) return rc;
   // the solve starts from primStage's fluid rows (guessInSolve); the field

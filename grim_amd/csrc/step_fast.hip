@@ -6,12 +6,15 @@
 //
 // Same mathematics as the exact kernels of step.hip, reorganised for fewer
 // instructions:
-//  * WENO5 (weno5.cpp:111-257) forms each face value with one division: the
-//    nonlinear weights c_k / beta_k^2 and their sum are scaled by
-//    16 beta_1^2 beta_2^2 beta_3^2, which leaves products of the betas;
-//  * each quotient family with a common divisor (1/u^0 in b^i, 1/|b| and
-//    1/b^2 in the stress rows, 1/tau and 1/(rho + Gamma u) in the speeds,
-//    1/(2A) for the two roots) takes one reciprocal;
+//  * WENO5 (weno5.cpp:111-257) forms both face values of a zone from one set
+//    of smoothness indicators, each with one division: the nonlinear weights
+//    c_k / beta_k^2 and their sum are scaled by beta_1^2 beta_2^2 beta_3^2,
+//    which leaves products of the betas;
+//  * T^mu_nu is A^mu u_nu + C^mu b_nu + delta^mu_nu E, of which only the rows
+//    and components that enter a result are formed, with shared reciprocals
+//    (1/u^0, 1/|b|, 1/(rho + Gamma u), 1/(2A) for the two speeds);
+//  * the closure enters fluxes and sources through chi/tau and nu/tau, in
+//    which tau cancels;
 //  * the characteristic speeds read the inverse metric entries the unit
 //    covectors pick instead of contracting with zeros;
 //  * the sources read the 40 symmetric connection planes once, in one pass
@@ -72,152 +75,6 @@ __device__ __forceinline__ void faceValues(const double* y, double theta, double
     weno5Fast(y, left, right);
   else
     reconstructZone<RECON>(y, theta, left, right);
-}
-
-// fluidElement::set's kinematics (physics.cpp:60-116) with one reciprocal of
-// u^0 for the three b^i.
-template <class L>
-__device__ __forceinline__ void kinematicsFast(const double* P, const ZoneGeom& G, const DevParams& prm,
-                                               Kinematics& k) {
-  k.rho = smax(P[RHO], prm.rhoFloor);
-  k.u = smax(P[UU], prm.uFloor);
-  const double u1 = P[U1], u2 = P[U2], u3 = P[U3];
-  const double B1 = P[L::B1], B2 = P[L::B2], B3 = P[L::B3];
-  k.pressure = (prm.gam - 1.) * k.u;
-  k.temperature = smax(fastDiv(k.pressure, k.rho), prm.tFloor);
-  const double gamma = sqrt(1. + G.cov(1, 1) * u1 * u1 + G.cov(2, 2) * u2 * u2 + G.cov(3, 3) * u3 * u3 +
-                            2. * (G.cov(1, 2) * u1 * u2 + G.cov(1, 3) * u1 * u3 + G.cov(2, 3) * u2 * u3));
-  k.gammaLF = gamma;
-  k.uCon[0] = fastDiv(gamma, G.alpha);
-  const double invU0 = fastDiv(G.alpha, gamma);
-  const double ga = gamma * G.alpha;
-  k.uCon[1] = u1 - ga * G.gcon0[1];
-  k.uCon[2] = u2 - ga * G.gcon0[2];
-  k.uCon[3] = u3 - ga * G.gcon0[3];
-#pragma unroll
-  for (int mu = 0; mu < 4; mu++)
-    k.uCov[mu] = G.cov(mu, 0) * k.uCon[0] + G.cov(mu, 1) * k.uCon[1] + G.cov(mu, 2) * k.uCon[2] +
-                 G.cov(mu, 3) * k.uCon[3];
-  k.bCon[0] = B1 * k.uCov[1] + B2 * k.uCov[2] + B3 * k.uCov[3];
-  k.bCon[1] = (B1 + k.bCon[0] * k.uCon[1]) * invU0;
-  k.bCon[2] = (B2 + k.bCon[0] * k.uCon[2]) * invU0;
-  k.bCon[3] = (B3 + k.bCon[0] * k.uCon[3]) * invU0;
-#pragma unroll
-  for (int mu = 0; mu < 4; mu++)
-    k.bCov[mu] = G.cov(mu, 0) * k.bCon[0] + G.cov(mu, 1) * k.bCon[1] + G.cov(mu, 2) * k.bCon[2] +
-                 G.cov(mu, 3) * k.bCon[3];
-  k.bSqr = k.bCon[0] * k.bCov[0] + k.bCon[1] * k.bCov[1] + k.bCon[2] * k.bCov[2] + k.bCon[3] * k.bCov[3] +
-           prm.bSqrFloor;
-}
-
-// setFluidElementParameters and the rescaled q, deltaP of set() (physics.cpp:
-// 118-151; torus closure torus/problem.cpp:7-55), the element's closure with
-// unit alphas, as elementClosure.
-template <class L>
-__device__ __forceinline__ void closureFast(const double* P, const Kinematics& k, const DevParams& prm,
-                                            double radius, Closure& c) {
-  const double cs2 = fastDiv(prm.gam * k.pressure, k.rho + prm.gam * k.u);
-  c.soundSpeed = sqrt(cs2);
-  c.bNorm = sqrt(k.bSqr);
-  c.q = 0.;
-  c.deltaP = 0.;
-  c.tau = c.chi = c.nu = 0.;
-  if constexpr (L::EMHD) {
-    const double aC = prm.condAlpha, aV = prm.viscAlpha;
-    if constexpr (L::COND_ON)
-      c.q = prm.highOrderCond ? P[L::Q] * k.temperature * sqrt(k.rho * aC * cs2) : P[L::Q];
-    if constexpr (L::VISC_ON)
-      c.deltaP = prm.highOrderVisc ? P[L::DP] * sqrt(k.temperature * k.rho * aV * cs2) : P[L::DP];
-    if (prm.closure == GRIM_CLOSURE_LINEAR_MODES) {
-      c.tau = 1.0;
-      c.chi = cs2;
-      c.nu = cs2;
-    } else if (prm.closure == GRIM_CLOSURE_SHOCK_TESTS) {
-      c.tau = 0.1;
-      c.chi = prm.condAlpha * cs2 * c.tau;
-      c.nu = prm.viscAlpha * cs2 * c.tau;
-    } else if (prm.closure == GRIM_CLOSURE_BUOYANCY) {
-      c.chi = sqrt(radius);
-      c.tau = fastDiv(1.2 * c.chi, cs2);
-    } else {
-      const double dyn = radius * sqrt(radius);
-      double tau = dyn;
-      const double cs3 = cs2 * c.soundSpeed;
-      if constexpr (L::COND_ON) {
-        double y = fastDiv(fabs(c.q), prm.condClosureFactor * k.rho * cs3);
-        y = exp((1. - y) * 100.);
-        tau = smin(tau, dyn * (fastDiv(y, y + 1.) + 1.e-5));
-      }
-      if constexpr (L::VISC_ON) {
-        const double p = k.pressure, dP = c.deltaP, bs = k.bSqr;
-        const double dPmod = fastDiv(smax(p - (2. / 3.) * dP, prm.bSqrFloor), smax(p + (1. / 3.) * dP, prm.bSqrFloor));
-        const double dPmaxPlus = smin(prm.viscClosureFactor * bs * 0.5 * dPmod, (1.49 / 1.07) * p);
-        const double dPmaxMinus = smax(-prm.viscClosureFactor * bs, (-2.99 / 1.07) * p);
-        const double dPmax = (dP > 0.) ? dPmaxPlus : dPmaxMinus;
-        double y = fastDiv(fabs(dP), fabs(dPmax) + prm.bSqrFloor);
-        y = exp((1. - y) * 100.);
-        tau = smin(tau, dyn * (fastDiv(y, y + 1.) + 1.e-5));
-      }
-      c.tau = tau;
-      const double maxAlpha = fastDiv(1. - cs2, 2. * cs2 + 1.e-12);
-      c.chi = smin(maxAlpha, prm.condAlpha) * cs2 * c.tau;
-      c.nu = smin(maxAlpha, prm.viscAlpha) * cs2 * c.tau;
-    }
-  }
-}
-
-// Reciprocals every stress row shares.
-struct StressInv {
-  double qOverB;   // q / |b|
-  double dPOverB2; // deltaP / b^2
-};
-
-template <class L>
-__device__ __forceinline__ StressInv stressInv(const Kinematics& k, const Closure& c) {
-  StressInv s{0., 0.};
-  if constexpr (L::COND_ON) s.qOverB = fastDiv(c.q, c.bNorm);
-  if constexpr (L::VISC_ON) s.dPOverB2 = fastDiv(c.deltaP, k.bSqr);
-  return s;
-}
-
-// Row MU of T^mu_nu (physics.cpp:153-178).
-template <class L, int MU>
-__device__ __forceinline__ void stressRowFast(const Kinematics& k, const Closure& c, const StressInv& si,
-                                              double* T) {
-  const double w = k.rho + k.u + k.pressure + k.bSqr;
-  const double wu = w * k.uCon[MU];
-#pragma unroll
-  for (int nu = 0; nu < 4; nu++) {
-    double t = wu * k.uCov[nu] - k.bCon[MU] * k.bCov[nu];
-    if (MU == nu) t += k.pressure + 0.5 * k.bSqr;
-    if constexpr (L::COND_ON) t += si.qOverB * (k.uCon[MU] * k.bCov[nu] + k.bCon[MU] * k.uCov[nu]);
-    if constexpr (L::VISC_ON)
-      t += -si.dPOverB2 * (k.bCon[MU] * k.bCov[nu]) +
-           (c.deltaP * (1. / 3.)) * ((MU == nu ? 1. : 0.) + k.uCon[MU] * k.uCov[nu]);
-    T[nu] = t;
-  }
-}
-
-// fluidElement::computeFluxes(DIR) (physics.cpp:185-217); DIR = 0 gives U.
-template <class L, int DIR>
-__device__ __forceinline__ void fluxesFast(const double* P, const Kinematics& k, const Closure& c,
-                                           const StressInv& si, double g, double* F) {
-  double T[4];
-  stressRowFast<L, DIR>(k, c, si, T);
-  const double gu = g * k.uCon[DIR];
-  F[RHO] = gu * k.rho;
-  F[UU] = g * T[0] + F[RHO];
-  F[U1] = g * T[1];
-  F[U2] = g * T[2];
-  F[U3] = g * T[3];
-  // the component along DIR is b^d u^d - b^d u^d = 0 exactly, as grim
-  // computes it (a contracted b^d u^d - b^d u^d would leave the product's
-  // rounding error)
-#pragma unroll
-  for (int c = 1; c <= 3; c++)
-    F[L::B1 + c - 1] = (c == DIR) ? 0. : g * (k.bCon[c] * k.uCon[DIR] - k.bCon[DIR] * k.uCon[c]);
-  if constexpr (L::COND_ON) F[L::Q] = gu * P[L::Q];
-  if constexpr (L::VISC_ON) F[L::DP] = gu * P[L::DP];
 }
 
 // The geometry one side of a face needs: the zone geometry, the inverse
@@ -597,165 +454,241 @@ __host__ __device__ constexpr int sym4(int k, int m) {
   return (k < m ? k : m) * 4 - ((k < m ? k : m) * ((k < m ? k : m) + 1)) / 2 + (k < m ? m : k);
 }
 
-// computeExplicitSources (physics.cpp:360-586) for the bulk zones of box:
-// one pass over the connection's upper index l, whose 10 symmetric planes
-// feed the geometric source -g T^k_l Gamma^l_{k n} and the covariant
-// derivative u_{mu;nu} = d_nu u_mu - Gamma^l_{nu mu} u_l; the old implicit
-// sources with the stage element's tau; on the half stage consOld.
+// The zone of this thread when the planes of a box are dealt to the 8 XCDs in
+// bands of X2 rows (workgroups go round the XCDs in turn): the X2 and X3
+// neighbours of a zone and its geometry column, which every X3 plane reads
+// again, then stay in one XCD's L2 (sourcesFastKernel on 192x192x128 EMHD
+// zones: 1.33 to 1.04 GB from beyond the L2, 529 to 500 us against workgroups
+// in memory order).
+__device__ __forceinline__ bool bandZone(const Box& box, int& i, int& j, int& k) {
+  const unsigned ni = (unsigned)(box.hi[0] - box.lo[0]), nk = (unsigned)(box.hi[2] - box.lo[2]);
+  const unsigned plane = ni * (unsigned)(box.hi[1] - box.lo[1]);
+  const unsigned x = blockIdx.x & 7u, t = (blockIdx.x >> 3) * (unsigned)kBlock + threadIdx.x;
+  const unsigned lo = plane / 8u * x + min(x, plane % 8u), size = plane / 8u + (x < plane % 8u ? 1u : 0u);
+  if (size == 0 || t >= size * nk) return false;
+  const unsigned r = lo + t % size;
+  i = box.lo[0] + (int)(r % ni);
+  j = box.lo[1] + (int)(r / ni);
+  k = box.lo[2] + (int)(t / size);
+  return true;
+}
+
+unsigned bandBlocks(const Box& b) {
+  const int64_t plane = (int64_t)(b.hi[0] - b.lo[0]) * (b.hi[1] - b.lo[1]);
+  return 8u * (unsigned)(((plane + 7) / 8 * (b.hi[2] - b.lo[2]) + kBlock - 1) / kBlock);
+}
+
+// computeExplicitSources (physics.cpp:360-586) for the bulk zones of box, the
+// old implicit sources with the stage element's tau and, on the half stage,
+// consOld, from the element in the form of faceElement.
+//
+// Nothing is held that is only contracted: each derivative d_nu u_mu and each
+// connection entry goes at once into the three scalars the EMHD sources read
+// (g^{mu nu}, b^mu b^nu and u^mu b^nu times u_{nu;mu}), and T^k_l is formed
+// for one l at a time from A^k u_l + C^k b_l + delta^k_l E.  tau cancels from
+// the sources of q and deltaP.
+//
+// sparseImp: only the q and deltaP rows of the old implicit sources are
+// written (the others are zero from the start).
+struct PerDir {
+  double v[3];
+};
+
 template <class L, int RECON>
-__global__ __launch_bounds__(kBlock) void sourcesFastKernel(StepArgs a, Box box, const double* __restrict__ prim,
-                                                            const double* __restrict__ primOld,
-                                                            const double* __restrict__ geomC,
-                                                            const double* __restrict__ gamma40,
-                                                            const double* __restrict__ uT, double* __restrict__ sExp,
-                                                            double* __restrict__ sImp, double* __restrict__ consOld) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= box.count()) return;
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) void sourcesFastKernel(
+    StepArgs a, PerDir inv12dX, Box box, const double* __restrict__ prim, const double* __restrict__ primOld,
+    const double* __restrict__ geomC, const double* __restrict__ gamma40, const double* __restrict__ uT,
+    double* __restrict__ sExp, double* __restrict__ sImp, double* __restrict__ consOld, int sparseImp) {
   int i, j, k;
-  box.at(t, i, j, k);
+  if (!bandZone(box, i, j, k)) return;
   const Dims& D = a.D;
-  const int64_t n = D.n, z = flatIndex(D, i, j, k);
-  const int64_t ng = D.ng, zg = geomIndex(D, i, j);
+  const int64_t n = D.n, ng = D.ng;
+  const uint32_t zb = (uint32_t)flatIndex(D, i, j, k) * 8u, zg = (uint32_t)geomIndex(D, i, j) * 8u;
+  const DevParams& prm = a.prm;
   double P[L::DOF];
 #pragma unroll
-  for (int v = 0; v < L::DOF; v++) P[v] = prim[v * n + z];
-  GeomFull G;
-  loadGeomFull(geomC, ng, zg, G);
-  Kinematics kk;
-  Closure cc;
-  kinematicsFast<L>(P, G.zg, a.prm, kk);
-  closureFast<L>(P, kk, a.prm, G.r, cc);
-  const StressInv si = stressInv<L>(kk, cc);
-  const double g = G.zg.g;
-  if (consOld) {
-    double U[L::DOF];
-    fluxesFast<L, 0>(P, kk, cc, si, g, U);
+  for (int v = 0; v < L::DOF; v++) P[v] = ldOff(prim + v * n, zb);
+  ZoneGeom G;
 #pragma unroll
-    for (int v = 0; v < L::DOF; v++) consOld[v * n + z] = U[v];
-  }
-  double src[L::NF];
+  for (int q = 0; q < 10; q++) G.gcov[q] = ldOff(geomC + q * ng, zg);
 #pragma unroll
-  for (int v = 0; v < L::NF; v++) src[v] = 0.;
-  const bool curved = a.metric != GRIM_METRIC_MINKOWSKI;
-  // T^k_l, k-major
-  double T[4][4];
-  if (curved) {
-    stressRowFast<L, 0>(kk, cc, si, T[0]);
-    stressRowFast<L, 1>(kk, cc, si, T[1]);
-    stressRowFast<L, 2>(kk, cc, si, T[2]);
-    stressRowFast<L, 3>(kk, cc, si, T[3]);
+  for (int q = 0; q < 4; q++) G.gcon0[q] = ldOff(geomC + (GEOM_GCON0 + q) * ng, zg);
+  G.alpha = ldOff(geomC + GEOM_ALPHA * ng, zg);
+  G.g = ldOff(geomC + GEOM_G * ng, zg);
+  // The stencils of u_0..u_3 and T along each direction, three ahead of their
+  // use.
+  constexpr int STENCILS = L::EMHD ? (L::COND_ON ? 15 : 12) : 0, RING = 4;
+  double y[RING][5];
+  int sB[3];  // no neighbours along a missing dimension: the zone itself
+#pragma unroll
+  for (int d = 0; d < 3; d++) sB[d] = d < D.dim ? (int)D.s[d] * 8 : 0;
+  auto loadStencil = [&](int e) {
+    if (e >= STENCILS) return;
+#pragma unroll
+    for (int q = 0; q < 5; q++)
+      if (q != 2 || RECON != GRIM_RECON_WENO5)
+        y[e % RING][q] = ldOff(uT + e / 3 * n, zb + (uint32_t)((q - 2) * sB[e % 3]));
+  };
+  double gam[2][10];
+  auto loadGamma = [&](int l) {
+#pragma unroll
+    for (int q = 0; q < 10; q++) gam[l & 1][q] = ldOff(gamma40 + (l * 10 + q) * ng, zg);
+  };
+#pragma unroll
+  for (int e = 0; e < RING - 1; e++) loadStencil(e);
+
+  const double rho = smax(P[RHO], prm.rhoFloor), u = smax(P[UU], prm.uFloor);
+  const double *ut = P + U1, *B = P + L::B1;
+  const double p = (prm.gam - 1.) * u, g = G.g;
+  double uc[4], uCov[4], bc[4], bCov[4];
+  lower3(G, ut, uCov + 1);
+  lower3(G, B, bCov + 1);
+  const double lor = fastSqrt(1. + dot3(ut, uCov + 1));
+  const double invU0 = fastDiv(G.alpha, lor), ga = lor * G.alpha;
+  uc[0] = fastDiv(lor, G.alpha);
+  uCov[0] = G.cov(0, 1) * ut[0] + G.cov(0, 2) * ut[1] + G.cov(0, 3) * ut[2] - ga;
+  const double b0 = dot3(B, uCov + 1);
+  const double bsq = (dot3(B, bCov + 1) + b0 * b0) * invU0 * invU0 + prm.bSqrFloor;
+  bc[0] = b0;
+  bCov[0] = (G.cov(0, 1) * B[0] + G.cov(0, 2) * B[1] + G.cov(0, 3) * B[2] + b0 * uCov[0]) * invU0;
+#pragma unroll
+  for (int q = 1; q < 4; q++) {
+    uc[q] = ut[q - 1] - ga * G.gcon0[q];
+    bc[q] = (B[q - 1] + b0 * uc[q]) * invU0;
+    bCov[q] = (bCov[q] + b0 * uCov[q]) * invU0;
   }
-  double graduCov[4][4];
+  const double w = rho + u + p + bsq;
+  double A[4], C[4], E = p + 0.5 * bsq, T = 0., ib = 0.;
+  FastClosure cl{1., 0., 0.};
+  double qb = 0., third = 0., dPb = 0.;
   if constexpr (L::EMHD) {
-    auto slopeOf = [&](const double* arr, int d) {
-      double y[5];
+    T = smax(p * fastRcp(rho), prm.tFloor);
+    ib = fastRsqrt(bsq);
+    const double r = ldOff(geomC + LOC_R * ng, zg);
+    fastClosure<L>(rho, u, p, T, bsq, L::COND_ON ? P[L::Q] : 0., L::VISC_ON ? P[L::DP] : 0., prm, 1., 1., r, cl);
+    const double cs2 = prm.gam * p * fastRcp(rho + prm.gam * u);
+    if constexpr (L::COND_ON)
+      qb = (prm.highOrderCond ? P[L::Q] * T * fastSqrt(rho * prm.condAlpha * cs2) : P[L::Q]) * ib;
+    if constexpr (L::VISC_ON) {
+      const double dP = prm.highOrderVisc ? P[L::DP] * fastSqrt(T * rho * prm.viscAlpha * cs2) : P[L::DP];
+      third = dP * (1. / 3.);
+      dPb = dP * ib * ib;
+    }
+    E = E + third;
+  }
 #pragma unroll
-      for (int q = 0; q < 5; q++) y[q] = arr[z + (q - 2) * D.s[d]];
-      return slopeZone<RECON>(y, a.theta, a.dX[d]);
-    };
+  for (int q = 0; q < 4; q++) {
+    A[q] = w * uc[q] + qb * bc[q] + third * uc[q];
+    C[q] = qb * uc[q] - bc[q] - dPb * bc[q];
+  }
+  if (consOld) {
+    stOff(consOld, zb, g * (rho * uc[0]));
+    stOff(consOld + UU * n, zb, g * (A[0] * uCov[0] + C[0] * bCov[0] + E + rho * uc[0]));
 #pragma unroll
-    for (int mu = 0; mu < 4; mu++) {
-      const double* um = uT + mu * n;
-      graduCov[0][mu] = 0.;
-      graduCov[1][mu] = slopeOf(um, 0);
-      graduCov[2][mu] = D.dim > 1 ? slopeOf(um, 1) : 0.;
-      graduCov[3][mu] = D.dim > 2 ? slopeOf(um, 2) : 0.;
+    for (int q = 1; q < 4; q++) stOff(consOld + (UU + q) * n, zb, g * (A[0] * uCov[q] + C[0] * bCov[q]));
+    if constexpr (L::COND_ON) stOff(consOld + L::Q * n, zb, g * (uc[0] * P[L::Q]));
+    if constexpr (L::VISC_ON) stOff(consOld + L::DP * n, zb, g * (uc[0] * P[L::DP]));
+#pragma unroll
+    for (int q = 0; q < 3; q++) stOff(consOld + (L::B1 + q) * n, zb, g * B[q]);
+  }
+  if constexpr (L::EMHD) {
+    if (sImp) {
+      const double gt = g * fastRcp(cl.tau);
+#pragma unroll
+      for (int v = 0; v < L::NF; v++) {
+        const bool row = (L::VISC_ON && v == L::DP) || (L::COND_ON && v == L::Q);
+        if (row)
+          stOff(sImp + v * n, zb, gt * ldOff(primOld + v * n, zb));
+        else if (!sparseImp)
+          stOff(sImp + v * n, zb, 0.);
+      }
     }
   }
+
+  // g^{mu nu}, b^mu b^nu and u^mu b^nu times u_{nu;mu}; b^mu d_mu T
+  double div = 0., bb = 0., ub = 0., bT = 0.;
+  double gcon[10];  // g^{mu nu}, packed as sym4
+  if constexpr (L::EMHD) {
+#pragma unroll
+    for (int q = 0; q < 4; q++) gcon[q] = G.gcon0[q];
+#pragma unroll
+    for (int q = 0; q < 6; q++) gcon[4 + q] = ldOff(geomC + (16 + q) * ng, zg);
+#pragma unroll
+    for (int e = 0; e < STENCILS; e++) {
+      loadStencil(e + RING - 1);
+      const int m = e / 3, d = e % 3;
+      const double* f = y[e % RING];
+      double s;
+      if constexpr (RECON == GRIM_RECON_WENO5)  // central differences (weno5.cpp:52-65)
+        s = ((f[0] - f[4]) + 8. * (f[3] - f[1])) * inv12dX.v[d];
+      else
+        s = slopeZone<RECON>(f, a.theta, a.dX[d]);
+      if (d >= D.dim) s = 0.;
+      if (m < 4) {
+        div = div + gcon[sym4(d + 1, m & 3)] * s;
+        bb = bb + bc[d + 1] * bc[m & 3] * s;
+        ub = ub + uc[d + 1] * bc[m & 3] * s;
+      } else {
+        bT = bT + bc[d + 1] * s;
+      }
+      asm volatile("" : "+v"(div), "+v"(bb), "+v"(ub), "+v"(bT));
+    }
+  }
+  double src[4] = {0., 0., 0., 0.};
+  const bool curved = a.metric != GRIM_METRIC_MINKOWSKI;
   if (curved || L::EMHD) {
+    loadGamma(0);
 #pragma unroll
     for (int l = 0; l < 4; l++) {
-      double gam[10];
-#pragma unroll
-      for (int q = 0; q < 10; q++) gam[q] = gamma40[(l * 10 + q) * ng + zg];
+      if (l < 3) loadGamma(l + 1);
+      const double* ga4 = gam[l & 1];
       if (curved) {
+        double t[4];
 #pragma unroll
-        for (int nu = 0; nu < 4; nu++) {
-          double s = 0.;
-#pragma unroll
-          for (int kap = 0; kap < 4; kap++) s += T[kap][l] * gam[sym4(kap, nu)];
-          src[UU + nu] -= g * s;
-        }
-      }
-      if constexpr (L::EMHD) {
-        const double ul = kk.uCov[l];
+        for (int q = 0; q < 4; q++) t[q] = A[q] * uCov[l] + C[q] * bCov[l] + (q == l ? E : 0.);
 #pragma unroll
         for (int nu = 0; nu < 4; nu++)
 #pragma unroll
-          for (int mu = 0; mu < 4; mu++) graduCov[nu][mu] -= gam[sym4(nu, mu)] * ul;
+          for (int q = 0; q < 4; q++) src[nu] = src[nu] + t[q] * ga4[sym4(q, nu)];
       }
+      if constexpr (L::EMHD) {
+        double cd = 0., cb = 0., cu = 0.;
+#pragma unroll
+        for (int mu = 0; mu < 4; mu++) {
+          double vb = 0.;  // Gamma^l_{mu nu} b^nu
+#pragma unroll
+          for (int nu = 0; nu < 4; nu++) {
+            vb = vb + ga4[sym4(mu, nu)] * bc[nu];
+            if (nu >= mu) cd = cd + (nu > mu ? 2. : 1.) * gcon[sym4(mu, nu)] * ga4[sym4(mu, nu)];
+          }
+          cb = cb + bc[mu] * vb;
+          cu = cu + uc[mu] * vb;
+        }
+        div = div - cd * uCov[l];
+        bb = bb - cb * uCov[l];
+        ub = ub - cu * uCov[l];
+      }
+      asm volatile("" : "+v"(src[0]), "+v"(src[1]), "+v"(src[2]), "+v"(src[3]), "+v"(div), "+v"(bb), "+v"(ub));
     }
   }
-  if constexpr (L::EMHD) {
-    double divuCov = 0.;
+  stOff(sExp, zb, 0.);
 #pragma unroll
-    for (int mu = 0; mu < 4; mu++)
-#pragma unroll
-      for (int nu = 0; nu < 4; nu++) divuCov += G.con(mu, nu) * graduCov[mu][nu];
-    const double invTau = 1. / cc.tau;
-    if constexpr (L::VISC_ON) {
-      const double rn = kk.rho * cc.nu;
-      const double c3 = 3. * rn / kk.bSqr;
-      double bb = 0.;
-#pragma unroll
-      for (int mu = 0; mu < 4; mu++)
-#pragma unroll
-        for (int nu = 0; nu < 4; nu++) bb += kk.bCon[mu] * kk.bCon[nu] * graduCov[mu][nu];
-      double deltaP0 = -divuCov * rn + c3 * bb;
-      if (a.prm.highOrderVisc == 1) deltaP0 = deltaP0 * sqrt(cc.tau / (rn * kk.temperature));
-      double sd = -g * deltaP0 * invTau;
-      if (a.prm.highOrderVisc == 1) sd -= 0.5 * g * divuCov * P[L::DP];
-      src[L::DP] = sd;
-    }
-    if constexpr (L::COND_ON) {
-      const double* Tp = uT + 4 * n;
-      double gradT[4];
-      gradT[0] = 0.;
-      {
-        double y[5];
-#pragma unroll
-        for (int q = 0; q < 5; q++) y[q] = Tp[z + (q - 2) * D.s[0]];
-        gradT[1] = slopeZone<RECON>(y, a.theta, a.dX[0]);
-      }
-      gradT[2] = 0.;
-      gradT[3] = 0.;
-      if (D.dim > 1) {
-        double y[5];
-#pragma unroll
-        for (int q = 0; q < 5; q++) y[q] = Tp[z + (q - 2) * D.s[1]];
-        gradT[2] = slopeZone<RECON>(y, a.theta, a.dX[1]);
-      }
-      if (D.dim > 2) {
-        double y[5];
-#pragma unroll
-        for (int q = 0; q < 5; q++) y[q] = Tp[z + (q - 2) * D.s[2]];
-        gradT[3] = slopeZone<RECON>(y, a.theta, a.dX[2]);
-      }
-      // q0 = -rho chi / |b| (b^mu d_mu T + T b^nu u^mu u_{nu;mu})
-      const double rcb = kk.rho * cc.chi / cc.bNorm;
-      double bgT = 0., buu = 0.;
-#pragma unroll
-      for (int mu = 0; mu < 4; mu++) {
-        bgT += kk.bCon[mu] * gradT[mu];
-#pragma unroll
-        for (int nu = 0; nu < 4; nu++) buu += kk.bCon[nu] * kk.uCon[mu] * graduCov[mu][nu];
-      }
-      double q0 = -rcb * (bgT + kk.temperature * buu);
-      if (a.prm.highOrderCond == 1) q0 = q0 * sqrt(cc.tau / (kk.rho * cc.chi)) / kk.temperature;
-      double sq = -g * q0 * invTau;
-      if (a.prm.highOrderCond == 1) sq -= 0.5 * g * divuCov * P[L::Q];
-      src[L::Q] = sq;
-    }
-    if (sImp) {
-#pragma unroll
-      for (int v = 0; v < L::NF; v++) sImp[v * n + z] = 0.;
-      const double gt = g * invTau;
-      if constexpr (L::VISC_ON) sImp[L::DP * n + z] = gt * primOld[L::DP * n + z];
-      if constexpr (L::COND_ON) sImp[L::Q * n + z] = gt * primOld[L::Q * n + z];
-    }
+  for (int nu = 0; nu < 4; nu++) stOff(sExp + (UU + nu) * n, zb, curved ? -g * src[nu] : 0.);
+  // q0 = -rho chi/|b| (b^mu d_mu T + T b^nu u^mu u_{nu;mu}) and deltaP0 =
+  // rho nu (3/b^2 b^mu b^nu u_{nu;mu} - u^mu_{;mu}), over tau; the high-order
+  // closure scales them by sqrt(tau/(rho chi))/T and sqrt(tau/(rho nu T))
+  if constexpr (L::COND_ON) {
+    const double rc = rho * cl.chiOverTau;
+    double s = g * ib * (bT + T * ub);
+    s = prm.highOrderCond == 1 ? s * fastSqrt(rc) * fastRcp(T) - 0.5 * g * div * P[L::Q] : s * rc;
+    stOff(sExp + L::Q * n, zb, s);
   }
-#pragma unroll
-  for (int v = 0; v < L::NF; v++) sExp[v * n + z] = src[v];
+  if constexpr (L::VISC_ON) {
+    const double rn = rho * cl.nuOverTau;
+    double s = g * (div - 3. * ib * ib * bb);
+    s = prm.highOrderVisc == 1 ? s * fastSqrt(fastDiv(rn, T)) - 0.5 * g * div * P[L::DP] : s * rn;
+    stOff(sExp + L::DP * n, zb, s);
+  }
 }
 
 __global__ __launch_bounds__(kBlock) void gamma40Kernel(int64_t n, const double* __restrict__ g64,
@@ -829,22 +762,24 @@ int launchFaceFast(const grim_params& p, const StepArgs& a, int dir, int recon, 
 
 int launchSourcesFast(const grim_params& p, const StepArgs& a, int recon, const Box& b, const double* prim,
                       const double* primOld, const double* geomC, const double* gamma40, const double* uT,
-                      double* sExp, double* sImp, double* consOld, hipStream_t s) {
+                      double* sExp, double* sImp, double* consOld, bool sparseImp, hipStream_t s) {
   GRIM_REQUIRE(planeOffsetsFit(a.D.n), "fast explicit stage: planes must hold fewer than 2^29 zones");
-  const unsigned nb = blocks(b.count(), kBlock);
+  const unsigned nb = bandBlocks(b);
+  PerDir c;
+  for (int d = 0; d < 3; d++) c.v[d] = 1. / (12. * a.dX[d]);
   return dispatchLayout(p, [&]<class L>() -> int {
     switch (recon) {
       case GRIM_RECON_WENO5:
-        sourcesFastKernel<L, GRIM_RECON_WENO5><<<nb, kBlock, 0, s>>>(a, b, prim, primOld, geomC, gamma40, uT, sExp,
-                                                                     sImp, consOld);
+        sourcesFastKernel<L, GRIM_RECON_WENO5><<<nb, kBlock, 0, s>>>(a, c, b, prim, primOld, geomC, gamma40, uT, sExp,
+                                                                     sImp, consOld, sparseImp);
         break;
       case GRIM_RECON_PPM:
-        sourcesFastKernel<L, GRIM_RECON_PPM><<<nb, kBlock, 0, s>>>(a, b, prim, primOld, geomC, gamma40, uT, sExp,
-                                                                   sImp, consOld);
+        sourcesFastKernel<L, GRIM_RECON_PPM><<<nb, kBlock, 0, s>>>(a, c, b, prim, primOld, geomC, gamma40, uT, sExp,
+                                                                   sImp, consOld, sparseImp);
         break;
       default:
-        sourcesFastKernel<L, GRIM_RECON_MINMOD><<<nb, kBlock, 0, s>>>(a, b, prim, primOld, geomC, gamma40, uT,
-                                                                      sExp, sImp, consOld);
+        sourcesFastKernel<L, GRIM_RECON_MINMOD><<<nb, kBlock, 0, s>>>(a, c, b, prim, primOld, geomC, gamma40, uT,
+                                                                      sExp, sImp, consOld, sparseImp);
     }
     return checkLaunch("sources (fast)");
   });

@@ -21,9 +21,11 @@ int launchFaceFast(const grim_params& p, const StepArgs& a, int dir, int recon, 
 
 // Explicit sources (geometric + EMHD gradients), the old implicit sources
 // and (consOld != NULL) the conserved variables of the bulk box b.
+// sparseImp: of the old implicit sources only the rows that can differ from
+// zero are written.
 int launchSourcesFast(const grim_params& p, const StepArgs& a, int recon, const Box& b, const double* prim,
                       const double* primOld, const double* geomC, const double* gamma40, const double* uT,
-                      double* sExp, double* sImp, double* consOld, hipStream_t s);
+                      double* sExp, double* sImp, double* consOld, bool sparseImp, hipStream_t s);
 
 // The symmetric connection: plane l*10 + (packed k <= n) of gamma40 takes
 // Gamma^l_{k n} of the 64-plane connection (plane l*16 + k*4 + n).
