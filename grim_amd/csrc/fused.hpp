@@ -159,28 +159,51 @@ __device__ __forceinline__ void fastClosure(double rho, double u, double p, doub
 // for the high-order closure, so no quotient by chi or nu is formed.  The
 // coefficient element is the old one when the caller passes the same planes
 // (grim's half step), which is evaluated once then.
+//
+// loadEmhdPlanes takes what it reads from memory, so that the caller can issue
+// those loads with its others.
+template <class L>
+struct EmhdPlanes {
+  double old[5], coef[L::DOF];  // elemOld's rho, u, u~^i; the coefficient element's primitives
+  double alphaC, alphaV, radius;
+};
+
+__device__ __forceinline__ bool coefIsOld(const grim_zone_batch& b) {
+  return !b.prim_coef || b.prim_coef == b.prim_old;
+}
+
+template <class L>
+__device__ __forceinline__ void loadEmhdPlanes(const grim_zone_batch& b, int64_t z, EmhdPlanes<L>& e) {
+  const int64_t n = b.n;
+  const double* coef = coefIsOld(b) ? b.prim_old : b.prim_coef;
+#pragma unroll
+  for (int v = 0; v < 5; v++) e.old[v] = b.prim_old[v * n + z];
+#pragma unroll
+  for (int v = 0; v < L::DOF; v++) e.coef[v] = coef[v * n + z];
+  e.alphaC = b.closure ? b.closure[z] : 1.;
+  e.alphaV = b.closure ? b.closure[n + z] : 1.;
+  e.radius = b.radius ? b.radius[batchGeomIndex(b, z)] : 0.;
+}
+
 template <class L>
 __device__ __forceinline__ void fusedEmhdConstants(const grim_zone_batch& b, const DevParams& prm, const ZoneGeom& G,
-                                                   int64_t z, double invDt, ZoneConst<L>& c, EmhdWeights& w) {
+                                                   const EmhdPlanes<L>& e, double invDt, ZoneConst<L>& c,
+                                                   EmhdWeights& w) {
 #pragma clang fp contract(on)
-  const int64_t n = b.n;
-  c.alphaC = b.closure ? b.closure[z] : 1.;
-  c.alphaV = b.closure ? b.closure[n + z] : 1.;
-  const double radius = b.radius ? b.radius[batchGeomIndex(b, z)] : 0.;
-  double P[L::DOF], utLow[3];
-#pragma unroll
-  for (int v = 0; v < L::DOF; v++) P[v] = b.prim_old[v * n + z];
-  double rho = smax(P[RHO], prm.rhoFloor), u = smax(P[UU], prm.uFloor);
+  c.alphaC = e.alphaC;
+  c.alphaV = e.alphaV;
+  const double radius = e.radius;
+  const double *old = e.old, *P = e.coef;
+  double utLow[3];
+  double rho = smax(old[RHO], prm.rhoFloor), u = smax(old[UU], prm.uFloor);
   double T = smax(fastDiv((prm.gam - 1.) * u, rho), prm.tFloor);
-  lower3(G, P + U1, utLow);
-  double lor = fastSqrt(1. + dot3(P + U1, utLow));
-  c.oldUCov[0] = G.cov(0, 1) * P[U1] + G.cov(0, 2) * P[U2] + G.cov(0, 3) * P[U3] - G.alpha * lor;
+  lower3(G, old + U1, utLow);
+  double lor = fastSqrt(1. + dot3(old + U1, utLow));
+  c.oldUCov[0] = G.cov(0, 1) * old[U1] + G.cov(0, 2) * old[U2] + G.cov(0, 3) * old[U3] - G.alpha * lor;
 #pragma unroll
   for (int i = 0; i < 3; i++) c.oldUCov[i + 1] = utLow[i];
   c.oldT = T;
-  if (b.prim_coef && b.prim_coef != b.prim_old) {
-#pragma unroll
-    for (int v = 0; v < L::DOF; v++) P[v] = b.prim_coef[v * n + z];
+  if (!coefIsOld(b)) {
     rho = smax(P[RHO], prm.rhoFloor);
     u = smax(P[UU], prm.uFloor);
     T = smax(fastDiv((prm.gam - 1.) * u, rho), prm.tFloor);

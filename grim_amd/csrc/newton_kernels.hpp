@@ -237,7 +237,7 @@ __device__ __forceinline__ bool newtonUpdate(double* P, const double* R, double 
   return accepted;
 }
 
-// Newton iterations of one zone, from its current primitives, for at most
+// Newton iterations of one zone, from the primitives P, for at most
 // `limit` updates (solve.cpp:10-200 read per zone: the zone stops when its
 // own sum R^2 <= atol).  Writes the primitives back; stats are stored, or
 // added to the earlier phase's when `accumulate`.  Once `budget` updates are
@@ -252,7 +252,7 @@ __device__ __forceinline__ bool solveZoneCore(const DevParams& prm, const grim_z
                                               const grim_newton_stats& st, int64_t z, int budget, int limit,
                                               int keep, bool accumulate, double dt, const ZoneGeom& G,
                                               const ZoneConst<L>& c, const ZoneScale& zs, const EmhdWeights& ew,
-                                              const double* start, const double* foldB, int& done);
+                                              double (&P)[L::DOF], int& done);
 
 // FOLDED: the zone's right-hand side, field rows and residual mask come from
 // the caller's registers (foldRhs, foldB, foldMask: the stage fold computed
@@ -285,6 +285,12 @@ __device__ __forceinline__ bool solveZone(const DevParams& prm, const grim_zone_
   const double dt = batchDt(b);
   ZoneGeom G;
   loadBatchGeom(b, z, G);
+  double P[L::DOF];
+  auto loadStart = [&] {
+#pragma unroll
+    for (int v = 0; v < L::DOF; v++)
+      P[v] = v < L::NF ? start[v * n + z] : (FOLDED ? foldB[v - L::NF] : b.prim[v * n + z]);
+  };
   ZoneConst<L> c;
   ZoneScale zs;
   EmhdWeights ew;
@@ -295,11 +301,20 @@ __device__ __forceinline__ bool solveZone(const DevParams& prm, const grim_zone_
     c.mask = maskZ;
   }
   if constexpr (ModeTraits<MODE>::fused) {
+    EmhdPlanes<L> planes;
+    if constexpr (L::EMHD) {
+      // every load of the zone is in flight before the constants of the first
+      // are formed
+      loadEmhdPlanes<L>(b, z, planes);
+      loadStart();
+      __builtin_amdgcn_sched_barrier(0);
+    }
     zoneScale(G, maskZ, dt, zs);
-    if constexpr (L::EMHD) fusedEmhdConstants<L>(b, prm, G, z, zs.invDt, c, ew);
+    if constexpr (L::EMHD) fusedEmhdConstants<L>(b, prm, G, planes, zs.invDt, c, ew);
   } else if constexpr (MODE == MODE_ANALYTIC64 && L::EMHD) {
     emhdWeights<L>(G, c, prm, dt, ew);
   }
+  if constexpr (!(ModeTraits<MODE>::fused && L::EMHD)) loadStart();
   if constexpr (kLdsState<L, MODE>) {
     static_assert(sizeof(ZoneGeom) <= kGeomSlot * sizeof(double) &&
                   sizeof(EmhdWeights) <= kWeightSlot * sizeof(double), "LDS slot sizes");
@@ -310,11 +325,10 @@ __device__ __forceinline__ bool solveZone(const DevParams& prm, const grim_zone_
         reinterpret_cast<EmhdWeights*>(zoneSlots + (size_t)kGeomSlot * blockDim.x + (size_t)kWeightSlot * threadIdx.x);
     *gs = G;
     *ws = ew;
-    return solveZoneCore<L, MODE, WIDE>(prm, b, st, z, budget, limit, keep, accumulate, dt, *gs, c, zs, *ws, start,
-                                        FOLDED ? foldB : nullptr, done);
+    return solveZoneCore<L, MODE, WIDE>(prm, b, st, z, budget, limit, keep, accumulate, dt, *gs, c, zs, *ws, P,
+                                        done);
   } else {
-    return solveZoneCore<L, MODE, WIDE>(prm, b, st, z, budget, limit, keep, accumulate, dt, G, c, zs, ew, start,
-                                        FOLDED ? foldB : nullptr, done);
+    return solveZoneCore<L, MODE, WIDE>(prm, b, st, z, budget, limit, keep, accumulate, dt, G, c, zs, ew, P, done);
   }
 }
 
@@ -323,13 +337,9 @@ __device__ __forceinline__ bool solveZoneCore(const DevParams& prm, const grim_z
                                               const grim_newton_stats& st, int64_t z, int budget, int limit,
                                               int keep, bool accumulate, double dt, const ZoneGeom& G,
                                               const ZoneConst<L>& c, const ZoneScale& zs, const EmhdWeights& ew,
-                                              const double* start, const double* foldB, int& done) {
+                                              double (&P)[L::DOF], int& done) {
   const int64_t n = b.n;
   const bool lead = !WIDE || (threadIdx.x % kWide) == 0;
-  double P[L::DOF];
-#pragma unroll
-  for (int v = 0; v < L::DOF; v++)
-    P[v] = v < L::NF ? start[v * n + z] : (foldB ? foldB[v - L::NF] : b.prim[v * n + z]);
 
   double R[L::NF];
   FusedPrimal f;

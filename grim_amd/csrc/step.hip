@@ -484,7 +484,11 @@ __global__ __launch_bounds__(kBlock) void foldKernel(StepArgs a, Box box, const 
   const int64_t n = D.n, z = flatIndex(D, i, j, k);
   if constexpr (!FOLD) {
 #pragma unroll
-    for (int v = 0; v < L::DOF; v++) divOut[v * n + z] = divergence<L, DIM>(D, a.dX, F, emf, v, z, i, j, a.fluxFilter);
+    for (int v = 0; v < L::DOF; v++) {
+      double f[DIM][2];
+      faceFluxes<L, DIM>(D, F, emf, v, z, f);
+      divOut[v * n + z] = divergence<DIM>(D, a.dX, v, i, j, a.fluxFilter, f);
+    }
   } else {
     double r[L::NF], B[3], rmax;
     foldZone<L, DIM>(D, a.dX, F, emf, geomC, consOld, sExp, sImp, *dtPrimeDev, z, i, j, a.fluxFilter, r, B, rmax);
