@@ -130,7 +130,7 @@ __device__ __forceinline__ double divergence(const Dims& D, const double* dX, in
 // with the divisions of one row between the loads of the next, a wavefront
 // waited out the memory latency some twenty times.  With the solve's own
 // loads batched likewise the EMHD phase 1 of 192x192x128 zones takes 845 us
-// instead of 917 (2.25 GB, 460 us at copy rate).
+// instead of 917: the 4.2 GB it moves take 860 us at the rate of a large copy.
 template <class L, int DIM, bool SPARSE_IMP = false>
 __device__ __forceinline__ void foldZone(const Dims& D, const double* dX, const double* __restrict__ F,
                                          const double* __restrict__ emf, const double* __restrict__ geomC,

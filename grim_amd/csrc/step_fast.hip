@@ -312,8 +312,8 @@ __device__ __forceinline__ void reconstructBoth(const StepArgs& a, const double*
 // rows (one more than the faces of a row) are numbered through; a wavefront
 // takes 63 of them and the one before.  Bound by FP64 issue (1,660
 // instructions per zone, about 210 us of 350 at 192x192x128 zones, EMHD; 510
-// with two threads per face) and by the 780 MB it moves; a fourth wavefront
-// per SIMD (blocks of 64) adds nothing.
+// with two threads per face) and by the 1.2 GB it moves (250 us at copy rate);
+// a fourth wavefront per SIMD (blocks of 64) adds nothing.
 constexpr int kRowBlock = 128;
 template <class L, int RECON>
 __global__ __launch_bounds__(kRowBlock) __attribute__((amdgpu_waves_per_eu(3))) void faceFluxRowKernel(
@@ -458,8 +458,8 @@ __host__ __device__ constexpr int sym4(int k, int m) {
 // bands of X2 rows (workgroups go round the XCDs in turn): the X2 and X3
 // neighbours of a zone and its geometry column, which every X3 plane reads
 // again, then stay in one XCD's L2 (sourcesFastKernel on 192x192x128 EMHD
-// zones: 1.33 to 1.04 GB from beyond the L2, 529 to 500 us against workgroups
-// in memory order).
+// zones: 500 us, 1.8 GB fetched from beyond the L2; 529 us with the workgroups
+// in memory order, which fetched 2.8 GB).
 __device__ __forceinline__ bool bandZone(const Box& box, int& i, int& j, int& k) {
   const unsigned ni = (unsigned)(box.hi[0] - box.lo[0]), nk = (unsigned)(box.hi[2] - box.lo[2]);
   const unsigned plane = ni * (unsigned)(box.hi[1] - box.lo[1]);
@@ -487,6 +487,11 @@ unsigned bandBlocks(const Box& b) {
 // (g^{mu nu}, b^mu b^nu and u^mu b^nu times u_{nu;mu}), and T^k_l is formed
 // for one l at a time from A^k u_l + C^k b_l + delta^k_l E.  tau cancels from
 // the sources of q and deltaP.
+//
+// 1,080 instructions instead of 1,670 and three wavefronts per SIMD instead of
+// two: 670 to 500 us on 192x192x128 EMHD zones (550 when two stencil fields
+// are loaded ahead instead of three directions, which spills).  Bound by the
+// 2.4 GB it moves, 480 us at the rate of a large copy.
 //
 // sparseImp: only the q and deltaP rows of the old implicit sources are
 // written (the others are zero from the start).
